@@ -32,6 +32,10 @@ constexpr int kDmaPerStage = 2;               // per wave: 1 x K + 1 x V (1 KiB 
 // Start cost of a piece in the work split, in keys (query staging and rotation,
 // page ids, the ring prologue).
 constexpr int kPieceCost = 256;
+// The same where the keys of a row group are split over the waves (a key takes
+// about 40 % less time there): 32 ragged sequences x 4 tokens, 1k - 8k keys, run
+// at 170 / 154 / 148.5 / 146.5 / 149 us with 128 / 256 / 400 / 512 / 768.
+constexpr int kPieceCostSplit = 512;
 
 static __device__ __align__(16) unsigned char zrow[512];
 
@@ -196,18 +200,26 @@ __device__ inline bool fill_page_cache(const DecodeParams& p, const int* bt, int
     return ok;
 }
 
+// Tokens of the largest row group of a launch (the token blocks of its merge).
+template <int RM>
+inline int max_group_tokens(const DecodeParams& p) {
+    const int n = RM == kRowVarlen ? p.T : p.S;
+    return n < kTokBlk ? n : kTokBlk;
+}
+
 __device__ inline uint32_t token_mask(int vis, int kb0) {
     const int lim = vis - kb0;
     return lim >= 32 ? 0xffffffffu : (lim <= 0 ? 0u : ((1u << lim) - 1u));
 }
 
-// Block (segment, token of the block): thread t -> head t/16, dims [(t%16)*8, +8).
+// Block (segment, token of the block; ntb tokens at most): thread t -> head t/16,
+// dims [(t%16)*8, +8).
 // A segment without pieces (no visible key) writes zeros, as the decode merge does.
 template <int DT, int RM>
-__global__ __launch_bounds__(256) void dv_merge_chunk(const DecodeParams p) {
+__global__ __launch_bounds__(256) void dv_merge_chunk(const DecodeParams p, int ntb) {
     using raw = typename Tr<DT>::raw;
-    const int sg = blockIdx.x / kTokBlk;
-    const int tb = blockIdx.x - sg * kTokBlk;
+    const int sg = blockIdx.x / ntb;
+    const int tb = blockIdx.x - sg * ntb;
     const int base = p.dir[2 * sg], cnt = p.dir[2 * sg + 1];
     if (cnt == 1) return;
     const int NHG = p.Hkv;

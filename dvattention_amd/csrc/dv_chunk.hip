@@ -241,10 +241,10 @@ __device__ inline void pv_tile(const VOp& v, const POperand& pB, Tile& t) {
 // Visibility of the 32 keys of the stage starting at kb0: the range end, and,
 // when some page of the sub-range is missing, page validity (a scalar branch
 // around a few instructions; the loop itself is not duplicated).
-template <int KVM, bool P2>
+template <int KVM, bool P2, int KS>
 __device__ inline uint32_t stage_mask(const DecodeParams& p, const Range& r, const int* pages, int sbnd, int kb0) {
     const int nin = sbnd - kb0;
-    uint32_t m = nin >= 32 ? 0xffffffffu : ((1u << nin) - 1u);
+    uint32_t m = nin >= 32 ? 0xffffffffu : ((1u << (KS > 1 && nin < 0 ? 0 : nin)) - 1u);  // KS > 1: stages past the end
     if (!r.pages_ok) {
         const int lane = threadIdx.x & 63;
         const bool kv_ok = row_of<KVM, P2>(p, r, pages, kb0 + (lane & 31)) >= 0;
@@ -333,6 +333,17 @@ __device__ inline void settle(POperand& a) {
     if constexpr (DT == kF16) asm volatile("" : "+v"(a.lo));
 }
 
+// Key split KS (1, 2 or 4): a row group of few tokens leaves waves without
+// tokens, and the arithmetic of 16 tokens per stage, not the loads, bound calls
+// of 2 .. 8 tokens.  So KS sets of kWaves / KS waves hold the same tokens and
+// take every KS-th stage: wave set kg computes stages kg, kg + KS, ... and one
+// step of the loop covers KS stages of the ring; the sets' tiles are combined
+// at the end of a piece (combine_split).  Steps in flight: the ring's steps
+// less one for KS = 1, every step of the ring for KS > 1.  32 sequences of
+// 4608 keys, 8 KV heads, bf16, same call without the split -> with it: 4 tokens
+// 194 -> 117 us (5.2 TB/s), 8 tokens 194 -> 131 us.
+template <int KS> constexpr int lead() { return KS == 1 ? kAhead : kStages / KS; }
+
 // Keys [sa, sbnd) of the current view for this wave's two tiles (A = tile 0,
 // B = tile 1): the stage loop.  Ring slot i % kStages holds stage i.  Per
 // stage i, in every wave:
@@ -343,10 +354,10 @@ __device__ inline void settle(POperand& a) {
 //          S_A(i+1) = K(i+1) Q_A^T and the loads of stage i+kAhead beside B's
 //          probabilities
 // so each wave's instruction stream alternates MFMAs of one tile with the
-// softmax of the other, and the two waves of a SIMD issue both at once.  A
-// slot is refilled (stage i+kAhead into the slot of stage i-1) only after the
-// barrier of stage i+1, which every wave reaches having completed its reads of
-// every stage <= i (the V reads of H1 are waited for before the barrier).  One
+// softmax of the other, and the two waves of a SIMD issue both at once.  The
+// loads of H2(i) refill slots of step i (KS > 1) or i-1 only: the barrier of
+// step i is reached by every wave with its reads of every stage <= i complete
+// (K(i) is read in H2(i-1), the V reads of H1 are waited for before the barrier).  One
 // K and one V^T operand set live in registers: K(i+1) is read after the MFMAs
 // of K(i) are issued, V(i) after those of V(i-1).  A's accumulators are
 // rescaled in H1 and written by MFMAs issued in H2 (and B's the other way
@@ -354,17 +365,19 @@ __device__ inline void settle(POperand& a) {
 // writes; mfma_settle before each softmax covers the MFMA -> VALU dependence
 // across the half-stage boundary.  Invisible keys get -inf scores only on a
 // partially visible stage (a uniform branch between the interleaved regions).
-template <int DT, int KVM, bool P2>
+template <int DT, int KVM, bool P2, int KS>
 __device__ inline void stream_range(const DecodeParams& p, const Range& r, const int* pages, unsigned char* smem,
-                                    int sa, int sbnd, const int (&vis_t)[kTiles], const u32x4 (&qB)[kTiles][4],
-                                    Tile (&tl)[kTiles]) {
+                                    int sa, int sbnd, int kg, const int (&vis_t)[kTiles],
+                                    const u32x4 (&qB)[kTiles][4], Tile (&tl)[kTiles]) {
+    constexpr int kLead = lead<KS>();
+    constexpr int kDma = kDmaPerStage * KS;  // loads per wave and step
     const uint32_t ring = lds_addr(smem);
-    const int nsteps = (sbnd - sa + kStep - 1) / kStep;
+    const int nsteps = (sbnd - sa + KS * kStep - 1) / (KS * kStep);
     const float l2 = p.l2scale;
-    // prologue: stages 0 .. kAhead-1 (past the end: rows of zeros)
+    // prologue: steps 0 .. kLead-1 (past the end: rows of zeros)
 #pragma unroll
-    for (int st = 0; st < kAhead; ++st) issue_stage<KVM, P2>(p, r, pages, ring, st, sa + st * kStep);
-    wait_vmcnt<kDmaPerStage * (kAhead - 1)>();  // own share of stage 0 landed
+    for (int st = 0; st < kLead * KS; ++st) issue_stage<KVM, P2>(p, r, pages, ring, st, sa + st * kStep);
+    wait_vmcnt<kDma * (kLead - 1)>();  // own share of step 0 landed
     wg_barrier();
 
     KOp kop;
@@ -373,13 +386,14 @@ __device__ inline void stream_range(const DecodeParams& p, const Range& r, const
     for (int cc = 0; cc < 8; ++cc) vop.v[cc] = u32x4{0u, 0u, 0u, 0u};  // the first P V adds 0 * 0
     f32x4 sa0, sa1, sb0, sb1;
     POperand pa = {}, pb = {};
-    read_k(smem, kop);
+    read_k(smem + kg * kStageBytes, kop);
     qk_tile<DT>(kop, qB[0], sa0, sa1);
 
     for (int i = 0; i < nsteps; ++i) {
-        const int kb0 = sa + i * kStep;
-        const unsigned char* slot = smem + (i % kStages) * kStageBytes;
-        const uint32_t okm = stage_mask<KVM, P2>(p, r, pages, sbnd, kb0);
+        const int st = i * KS + kg;  // this wave's stage of the step
+        const int kb0 = sa + st * kStep;
+        const unsigned char* slot = smem + (st % kStages) * kStageBytes;
+        const uint32_t okm = stage_mask<KVM, P2, KS>(p, r, pages, sbnd, kb0);
         const uint32_t mka = okm & token_mask(vis_t[0], kb0), mkb = okm & token_mask(vis_t[1], kb0);
         float pr[8];
         // ---- H1(i)
@@ -404,11 +418,19 @@ __device__ inline void stream_range(const DecodeParams& p, const Range& r, const
         }
         settle<DT>(pa);
         lds_wait();
-        wait_vmcnt<kDmaPerStage * (kAhead - 2)>();  // own share of stage i + 1 landed
+        wait_vmcnt<kDma * (kLead - 2)>();  // own share of step i + 1 landed
         wg_barrier();
-        // ---- H2(i) (stage i + 1 has landed even past the end -- rows of zeros --
+        if constexpr (KS > 1) {
+            // the loads of step i + kLead, into the slots of step i (free since the
+            // barrier): at once, as no later step is in flight when KS = 4; one
+            // stage at a time, the addresses of all do not fit the registers
+#pragma unroll 1
+            for (int q = (i + kLead) * KS; q < (i + kLead + 1) * KS; ++q)
+                issue_stage<KVM, P2>(p, r, pages, ring, q, sa + q * kStep);
+        }
+        // ---- H2(i) (step i + 1 has landed even past the end -- rows of zeros --
         // so K and S_A of the next stage need no branch; the last ones go unused)
-        read_k(smem + ((i + 1) % kStages) * kStageBytes, kop);
+        read_k(smem + ((st + KS) % kStages) * kStageBytes, kop);
         if (mkb != 0xffffffffu) mask_scores(sb0, sb1, mkb);
         mfma_settle(tl[1].o);
         pv_tile<DT>(vop, pa, tl[0]);
@@ -424,7 +446,7 @@ __device__ inline void stream_range(const DecodeParams& p, const Range& r, const
         pb = sm_finish<DT>(tl[1], pr);
         // the loads of stage i + kAhead (into the slot of stage i - 1, free since
         // the barrier), their address arithmetic beside the MFMAs
-        issue_stage<KVM, P2>(p, r, pages, ring, i + kAhead, sa + (i + kAhead) * kStep);
+        if constexpr (KS == 1) issue_stage<KVM, P2>(p, r, pages, ring, i + kLead, sa + (i + kLead) * kStep);
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
@@ -441,15 +463,69 @@ __device__ inline void stream_range(const DecodeParams& p, const Range& r, const
     __syncthreads();
 }
 
+// Key split: wave kg's tiles of the same tokens (kg = 0 .. KS - 1, waves
+// kg * kWaves/KS + tp) combined into those of kg = 0, through the idle ring:
+// lane by lane, O and the lane's row sum scaled to the common maximum (fp32).
+template <int KS>
+__device__ inline void combine_split(unsigned char* smem, int wv, int kg, int ntile, Tile (&tl)[kTiles]) {
+    constexpr int kPairs = kWaves / KS;  // waves per key subset
+    constexpr int kRec = 10 * 1024;      // per (wave, tile): 8 x 1 KiB of O, then m and l
+    static_assert((kWaves - kPairs) * kTiles * kRec <= kRingBytes + kPageCap * 4, "LDS of the combination");
+    const int lane = threadIdx.x & 63;
+    auto rec = [&](int k, int t) {  // record of tile t of the wave with subset k >= 1 of these tokens
+        return smem + (((k - 1) * kPairs + wv % kPairs) * kTiles + t) * kRec;
+    };
+    if (kg > 0) {
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) {
+            if (t >= ntile) continue;
+            unsigned char* b = rec(kg, t);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) *reinterpret_cast<f32x4*>(b + c * 1024 + lane * 16) = tl[t].o[c];
+            float* ml = reinterpret_cast<float*>(b + 8 * 1024);
+            ml[lane] = tl[t].m;
+            ml[64 + lane] = tl[t].l;
+        }
+    }
+    __syncthreads();
+    if (kg == 0) {
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) {
+            if (t >= ntile) continue;
+            float mk[KS], M = tl[t].m;
+#pragma unroll
+            for (int k = 1; k < KS; ++k) {
+                mk[k] = reinterpret_cast<const float*>(rec(k, t) + 8 * 1024)[lane];
+                M = fmaxf(M, mk[k]);
+            }
+            if (M == -DV_INF) continue;  // no visible key in any subset
+            const float s0 = __builtin_amdgcn_exp2f(tl[t].m - M);  // an empty subset (-inf) -> 0
+            tl[t].l *= s0;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) tl[t].o[c] *= s0;
+#pragma unroll
+            for (int k = 1; k < KS; ++k) {
+                const float sk = __builtin_amdgcn_exp2f(mk[k] - M);
+                tl[t].l += sk * reinterpret_cast<const float*>(rec(k, t) + 8 * 1024)[64 + lane];
+#pragma unroll
+                for (int c = 0; c < 8; ++c)
+                    tl[t].o[c] += sk * *reinterpret_cast<const f32x4*>(rec(k, t) + c * 1024 + lane * 16);
+            }
+            tl[t].m = M;
+        }
+    }
+    __syncthreads();  // the records are read before the ring is filled again
+}
+
 // One workgroup: keys [v0, v1) of row group rg for KV head hkv.
-template <int DT, int QM, int KVM, bool P2, int RM>
+template <int DT, int QM, int KVM, bool P2, int RM, int KS>
 __device__ void chunk_piece(const DecodeParams& p, unsigned char* smem, int* pages, int rg, int hkv, long long v0,
                             long long v1, bool final_out, int slot) {
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int g = lane >> 4, n = lane & 15;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Grp gr = group_of<RM>(p, rg);
     const int w = gr.w;
-    const int tok0 = wv * kTiles;  // this wave's first token of the group
+    const int kg = KS == 1 ? 0 : wv / (kWaves / KS);  // this wave's key subset
+    const int tok0 = (KS == 1 ? wv : wv % (kWaves / KS)) * kTiles;  // and first token of the group
     const int ntile = gr.ntok - tok0 < kTiles ? (gr.ntok - tok0 > 0 ? gr.ntok - tok0 : 0) : kTiles;
 
     Tile tl[kTiles];
@@ -513,12 +589,14 @@ __device__ void chunk_piece(const DecodeParams& p, unsigned char* smem, int* pag
                     const bool ok = fill_page_cache(p, p.bt + (long long)w * p.maxB, pages, r.lp0, lpl);
                     r.pages_ok = __syncthreads_and(ok) != 0;
                 }
-                stream_range<DT, KVM, P2>(p, r, pages, smem, sa, sbnd, vis_t, qB, tl);
+                stream_range<DT, KVM, P2, KS>(p, r, pages, smem, sa, sbnd, kg, vis_t, qB, tl);
             }
         }
         P += vis_blk;
         off += p.fl[f];
     }
+
+    if constexpr (KS > 1) combine_split<KS>(smem, wv, kg, ntile, tl);
 
     // epilogue: per tile, normalise and write the output or a partial slot
     {
@@ -526,7 +604,7 @@ __device__ void chunk_piece(const DecodeParams& p, unsigned char* smem, int* pag
     const int g = lane >> 4, n = lane & 15;
 #pragma unroll
     for (int t = 0; t < kTiles; ++t) {
-        if (t >= ntile) continue;
+        if (t >= ntile || kg > 0) continue;
         const float lt = rows4_sum(tl[t].l);
         const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
         const int h = hkv * kGqa + n;
@@ -540,7 +618,7 @@ __device__ void chunk_piece(const DecodeParams& p, unsigned char* smem, int* pag
                 *reinterpret_cast<u32x2*>(o + c * 16 + g * 4) = pk;
             }
         } else {
-            const int tb = wv * kTiles + t;  // token within the block
+            const int tb = tok0 + t;  // token within the block
             store_partial<DT>(p.part + (long long)slot * p.slot_floats, kTokBlk * kGqa, tb * kGqa + n, g, tl[t].o,
                               inv, lt > 0.0f ? tl[t].m + log2f(lt) : -DV_INF);
         }
@@ -550,7 +628,7 @@ __device__ void chunk_piece(const DecodeParams& p, unsigned char* smem, int* pag
 
 // P2: paged with a power-of-two block_size (shift and mask instead of a
 // division in the stage loop's row addressing).
-template <int DT, int QM, int KVM, bool P2, int RM>
+template <int DT, int QM, int KVM, bool P2, int RM, int KS>
 __global__ __launch_bounds__(kThreads) void dv_chunk(const DecodeParams p) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     // the ring starts at a 256-byte aligned LDS address (the XOR addressing of
@@ -563,7 +641,7 @@ __global__ __launch_bounds__(kThreads) void dv_chunk(const DecodeParams p) {
 
     run_schedule(p, NHG, s_pref, s_scan, [&](int rg) { return group_visible<KVM, RM>(p, rg); },
                  [&](int rg, int hg, long long v0, long long v1, bool fin, int slot, long long) {
-                     chunk_piece<DT, QM, KVM, P2, RM>(p, smem, pages, rg, hg, v0, v1, fin, slot);
+                     chunk_piece<DT, QM, KVM, P2, RM, KS>(p, smem, pages, rg, hg, v0, v1, fin, slot);
                  });
 }
 
@@ -667,11 +745,11 @@ __global__ __launch_bounds__(kVgThreads) void dv_varlen_groups(const int* cu, in
     }
 }
 
-template <int DT, int QM, int KVM, bool P2, int RM>
+template <int DT, int QM, int KVM, bool P2, int RM, int KS>
 hipError_t launch1(DecodeParams p, int device, int cus, long long cap, hipStream_t stream) {
     static std::atomic<unsigned long long> attr_done{0};
     hipError_t ea = once_per_device(attr_done, device, [] {
-        return hipFuncSetAttribute(reinterpret_cast<const void*>(&dv_chunk<DT, QM, KVM, P2, RM>),
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(&dv_chunk<DT, QM, KVM, P2, RM, KS>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(kMaxRows));
     });
     if (ea != hipSuccess) return ea;
@@ -679,22 +757,40 @@ hipError_t launch1(DecodeParams p, int device, int cus, long long cap, hipStream
     long long nwg = cus;  // one eight-wave workgroup per CU (LDS ring 96 KiB)
     if (nwg > cap) nwg = cap;
     p.nwg = nwg < 1 ? 1 : (int)nwg;
-    hipLaunchKernelGGL((dv_chunk<DT, QM, KVM, P2, RM>), dim3(p.nwg), dim3(kThreads), lds, stream, p);
+    hipLaunchKernelGGL((dv_chunk<DT, QM, KVM, P2, RM, KS>), dim3(p.nwg), dim3(kThreads), lds, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((dv_merge_chunk<DT, RM>), dim3(p.nrows * p.Hkv * kTokBlk), dim3(256), 0, stream, p);
+    const int ntb = max_group_tokens<RM>(p);
+    hipLaunchKernelGGL((dv_merge_chunk<DT, RM>), dim3(p.nrows * p.Hkv * ntb), dim3(256), 0, stream, p, ntb);
     return hipGetLastError();
 }
 
+template <int DT, int QM, int KVM, int RM, bool P2>
+hipError_t launch_split(const DecodeParams& p, int ks, int device, int cus, long long cap, hipStream_t stream) {
+    if (ks == 4) return launch1<DT, QM, KVM, P2, RM, 4>(p, device, cus, cap, stream);
+    if (ks == 2) return launch1<DT, QM, KVM, P2, RM, 2>(p, device, cus, cap, stream);
+    return launch1<DT, QM, KVM, P2, RM, 1>(p, device, cus, cap, stream);
+}
+
 template <int DT, int QM, int KVM, int RM>
-hipError_t launch(DecodeParams p, int device, int cus, long long cap, hipStream_t stream) {
+hipError_t launch(const DecodeParams& p, int ks, int device, int cus, long long cap, hipStream_t stream) {
     if constexpr (DT == kF32) {
         return launch_chunk32(QM, KVM, RM, p, device, cus, cap, stream);
     } else {
         if constexpr (KVM == kKvPaged)
-            if (p.bs_shift >= 0) return launch1<DT, QM, KVM, true, RM>(p, device, cus, cap, stream);
-        return launch1<DT, QM, KVM, false, RM>(p, device, cus, cap, stream);
+            if (p.bs_shift >= 0) return launch_split<DT, QM, KVM, RM, true>(p, ks, device, cus, cap, stream);
+        return launch_split<DT, QM, KVM, RM, false>(p, ks, device, cus, cap, stream);
     }
+}
+
+// Key split of a launch whose groups have at most ntok tokens: as many wave sets
+// as hold two tokens per wave.  (Eight sets for two tokens would take a ring step
+// of all eight stages, with nothing in flight beside it; two tokens run at 5.3
+// TB/s with four.)  A split step with no visible key must leave no trace in the
+// softmax, which -inf scores only do for a positive scale.
+int key_split(float l2scale, int ntok) {
+    if (!(l2scale > 0.0f) || ntok > 8) return 1;
+    return ntok > 4 ? 2 : 4;
 }
 
 }  // namespace chunk
@@ -734,7 +830,8 @@ hipError_t launch_groups(int dtype, int qmode, int kvmode, DecodeParams p, long 
     p.slot_floats = chunk::kTokBlk * kGqa * (kHeadDim + 1);
     p.part = reinterpret_cast<float*>(workspace);
     p.dir = reinterpret_cast<int*>(reinterpret_cast<unsigned char*>(workspace) + l.part);
-    p.piece_cost = chunk::kPieceCost;
+    const int ks = RM == kRowVarlen || dtype == kF32 ? 1 : chunk::key_split(p.l2scale, p.S);
+    p.piece_cost = ks == 1 ? chunk::kPieceCost : chunk::kPieceCostSplit;
     // odd workgroups (odd XCD of each pair) take shorter chunks, as in the decode
     // split; 30 per mille measured best on configuration 5
     static const int skew = env_per_mille("DVATTN_CHUNK_SKEW_PM", 30);
@@ -743,28 +840,28 @@ hipError_t launch_groups(int dtype, int qmode, int kvmode, DecodeParams p, long 
         p.row_begin = (int)g0;
         p.nrows = (int)(groups_total - g0 < kMaxRows ? groups_total - g0 : kMaxRows);
         const long long cap = ((long long)p.nrows * p.Hkv * max_keys_per_group + p.min_keys - 1) / p.min_keys;
-        if (RM == kRowVarlen) {
+        if constexpr (RM == kRowVarlen) {
             if (dtype == kBF16 && qmode == kQRotHalf && kvmode == kKvPaged)
-                e = chunk::launch<kBF16, kQRotHalf, kKvPaged, RM>(p, device, cus, cap, stream);
+                e = chunk::launch<kBF16, kQRotHalf, kKvPaged, RM>(p, ks, device, cus, cap, stream);
             else if (dtype == kF16 && qmode == kQRotHalf && kvmode == kKvPaged)
-                e = chunk::launch<kF16, kQRotHalf, kKvPaged, RM>(p, device, cus, cap, stream);
+                e = chunk::launch<kF16, kQRotHalf, kKvPaged, RM>(p, ks, device, cus, cap, stream);
             else if (dtype == kF32 && qmode == kQRotHalf && kvmode == kKvPaged)
-                e = chunk::launch<kF32, kQRotHalf, kKvPaged, RM>(p, device, cus, cap, stream);
+                e = chunk::launch<kF32, kQRotHalf, kKvPaged, RM>(p, ks, device, cus, cap, stream);
             else
                 e = hipErrorInvalidValue;
         } else {
             if (dtype == kBF16 && qmode == kQRotFull && kvmode == kKvPaged)
-                e = chunk::launch<kBF16, kQRotFull, kKvPaged, RM>(p, device, cus, cap, stream);
+                e = chunk::launch<kBF16, kQRotFull, kKvPaged, RM>(p, ks, device, cus, cap, stream);
             else if (dtype == kF16 && qmode == kQRotFull && kvmode == kKvPaged)
-                e = chunk::launch<kF16, kQRotFull, kKvPaged, RM>(p, device, cus, cap, stream);
+                e = chunk::launch<kF16, kQRotFull, kKvPaged, RM>(p, ks, device, cus, cap, stream);
             else if (dtype == kBF16 && qmode == kQPre && kvmode == kKvContig)
-                e = chunk::launch<kBF16, kQPre, kKvContig, RM>(p, device, cus, cap, stream);
+                e = chunk::launch<kBF16, kQPre, kKvContig, RM>(p, ks, device, cus, cap, stream);
             else if (dtype == kF16 && qmode == kQPre && kvmode == kKvContig)
-                e = chunk::launch<kF16, kQPre, kKvContig, RM>(p, device, cus, cap, stream);
+                e = chunk::launch<kF16, kQPre, kKvContig, RM>(p, ks, device, cus, cap, stream);
             else if (dtype == kF32 && qmode == kQRotFull && kvmode == kKvPaged)
-                e = chunk::launch<kF32, kQRotFull, kKvPaged, RM>(p, device, cus, cap, stream);
+                e = chunk::launch<kF32, kQRotFull, kKvPaged, RM>(p, ks, device, cus, cap, stream);
             else if (dtype == kF32 && qmode == kQPre && kvmode == kKvContig)
-                e = chunk::launch<kF32, kQPre, kKvContig, RM>(p, device, cus, cap, stream);
+                e = chunk::launch<kF32, kQPre, kKvContig, RM>(p, ks, device, cus, cap, stream);
             else
                 e = hipErrorInvalidValue;
         }

@@ -327,7 +327,8 @@ hipError_t launch1_f32(DecodeParams p, int device, int cus, long long cap, hipSt
     hipLaunchKernelGGL((dv_chunk32<QM, KVM, P2, RM>), dim3(p.nwg), dim3(kWaves32 * kWave), lds, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((dv_merge_chunk<kF32, RM>), dim3(p.nrows * p.Hkv * kTokBlk), dim3(256), 0, stream, p);
+    const int ntb = max_group_tokens<RM>(p);
+    hipLaunchKernelGGL((dv_merge_chunk<kF32, RM>), dim3(p.nrows * p.Hkv * ntb), dim3(256), 0, stream, p, ntb);
     return hipGetLastError();
 }
 

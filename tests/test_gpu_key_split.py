@@ -1,0 +1,39 @@
+"""Paged and contiguous calls of 2 .. 9 query tokens per sequence against the
+oracle: row groups whose keys are split over the waves of a workgroup (two or
+four wave sets, dvattention_amd/csrc/dv_chunk.hip) and the first size past it.
+Lengths end inside the first stage, the first step of a split and a later one,
+so some wave sets see no key; ragged batches also leave pieces of a few keys to
+merge.  Tolerances: test_gpu_parity.close."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import dvattn_oracle as O
+from test_gpu_parity import close, dv, rand_paged, run_paged  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("S", [2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("W,Hkv,bs,lens", [(2, 1, 16, [1]), (3, 2, 16, [33, 5]), (1, 4, 24, [128, 97]),
+                                           (5, 8, 16, [1500]), (2, 2, 32, [700, 0, 261])])
+def test_paged_few_tokens(dv, gpu, dtype, S, W, Hkv, bs, lens):  # noqa: F811
+    F = len(lens)
+    rng = np.random.default_rng(17 * S + sum(lens))
+    loc = rng.integers(-1, max(lens), size=(F, W, 1)) - S + 1 + np.arange(S)  # causal, some rows see no key
+    d = rand_paged(F, W, S, Hkv, bs, lens, 64, dtype, seed=S + bs, loc=loc, k_scale=2.0)
+    close(run_paged(dv, d, 0.1, gpu), O.paged_sdpa(0.1, **d), dtype, f"S={S}")
+
+
+@pytest.mark.parametrize("S", [2, 4, 7])
+def test_contiguous_few_tokens(dv, gpu, S):  # noqa: F811
+    F, W, Hkv, Ls = 2, 3, 2, [300, 45]
+    g = torch.Generator().manual_seed(S)
+    q = torch.randn(F, W, 16 * Hkv, S, 128, generator=g).to(torch.bfloat16)
+    ks = [torch.randn(W, Hkv, L, 128, generator=g).to(torch.bfloat16) for L in Ls]
+    vs = [torch.randn(W, Hkv, L, 128, generator=g).to(torch.bfloat16) for L in Ls]
+    loc = torch.from_numpy(np.random.default_rng(S).integers(-1, 310, size=(F, W, S)).astype(np.int32))
+    fl = torch.tensor(Ls, dtype=torch.int32)
+    out = dv.dvattn_sdpa(q.to(gpu), loc.to(gpu), [k.to(gpu) for k in ks], [v.to(gpu) for v in vs], 0.1, fl.to(gpu))
+    close(out, O.contig_sdpa(0.1, loc, q, fl, ks, vs), torch.bfloat16, f"S={S}")
