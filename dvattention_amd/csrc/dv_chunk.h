@@ -21,6 +21,7 @@ constexpr int kThreads = kWaves * kWave;
 constexpr int kTiles = 2;                     // 16-head query tiles (tokens) per wave
 constexpr int kHalf = kTiles / 2;             // tiles per MFMA/VALU group
 constexpr int kTokBlk = kWaves * kTiles;      // tokens per row group
+constexpr int kFewTok = 4;                    // tokens of a group whose keys are split four ways
 constexpr int kStages = 8;                    // K/V ring depth
 constexpr int kKvBytes = kStep * 256;         // one K (or V) stage tile: 32 keys x 256 B
 constexpr int kStageBytes = 2 * kKvBytes;     // K tile then V tile
@@ -170,34 +171,50 @@ __device__ inline long long group_visible(const DecodeParams& p, int rg) {
     return total;
 }
 
-// Page-cache fill of a chunk workgroup (kThreads threads): pages[i] = entry
-// lp0 + i of the sequence's block_tables row bt, for i < kPageCap (-1 past the
-// row or outside [0, num_blocks)).  Each thread issues all of its loads (on
+// Page-cache fill of a chunk workgroup (kThreads threads), in two parts so that
+// other loads can be issued between: pages[i] = entry lp0 + i of the sequence's
+// block_tables row bt, for the entries up to logical page lpl (-1 past the row or
+// outside [0, num_blocks)).  fetch_pages issues all of a thread's loads (on
 // clamped, in-bounds indices) before the first is waited for, where a strided
-// loop waited once per pass.  Returns whether this thread's entries up to
-// logical page lpl are all valid.
-__device__ inline bool fill_page_cache(const DecodeParams& p, const int* bt, int* pages, uint32_t lp0, uint32_t lpl) {
-    constexpr int kIt = kPageCap / kThreads;
-    static_assert(kIt * kThreads == kPageCap, "page cache entries per thread");
-    const int tid = threadIdx.x;
+// loop waited once per pass; store_pages returns whether this thread's entries
+// are all valid.
+constexpr int kPageIt = kPageCap / kThreads;
+static_assert(kPageIt * kThreads == kPageCap, "page cache entries per thread");
+
+__device__ inline void fetch_pages(const DecodeParams& p, const int* bt, uint32_t lp0, uint32_t lpl,
+                                   int (&pg)[kPageIt]) {
     const uint32_t maxB = (uint32_t)p.maxB;
-    int pg[kIt];
 #pragma unroll
-    for (int k = 0; k < kIt; ++k) {
-        const uint32_t lp = lp0 + (uint32_t)(tid + k * kThreads);
+    for (int k = 0; k < kPageIt; ++k) {
         pg[k] = -1;
-        if (maxB > 0) pg[k] = bt[lp < maxB ? lp : maxB - 1];
+        if (maxB > 0 && lp0 + (uint32_t)(k * kThreads) <= lpl) {  // uniform
+            const uint32_t lp = lp0 + (uint32_t)(threadIdx.x + k * kThreads);
+            pg[k] = bt[lp < maxB ? lp : maxB - 1];
+        }
     }
+}
+
+__device__ inline bool store_pages(const DecodeParams& p, int* pages, uint32_t lp0, uint32_t lpl,
+                                   const int (&pg)[kPageIt]) {
     bool ok = true;
 #pragma unroll
-    for (int k = 0; k < kIt; ++k) {
-        const uint32_t lp = lp0 + (uint32_t)(tid + k * kThreads);
-        int v = lp < maxB ? pg[k] : -1;
+    for (int k = 0; k < kPageIt; ++k) {
+        const uint32_t lp = lp0 + (uint32_t)(threadIdx.x + k * kThreads);
+        int v = lp < (uint32_t)p.maxB ? pg[k] : -1;
         if (v < 0 || v >= p.nblocks) v = -1;
-        pages[tid + k * kThreads] = v;
+        pages[threadIdx.x + k * kThreads] = v;
         if (lp <= lpl && v < 0) ok = false;
     }
     return ok;
+}
+
+// A wave-uniform value computed per lane, moved to scalar registers.
+__device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ inline long long uniform(long long v) {
+    const unsigned long long u = (unsigned long long)v;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+    return (long long)(((unsigned long long)hi << 32) | lo);
 }
 
 // Tokens of the largest row group of a launch (the token blocks of its merge).

@@ -91,85 +91,111 @@ struct Tile {
 // the token's full-width row, or its half-width varlen row; separately rounded
 // fp32 products and sum, rounded to the storage type; dims >= R untouched),
 // then lane (g, n) reads Q[n][c*32 + g*8 + 0..7] of every tile.  Wave-private
-// LDS region: 8 KiB.
-template <int DT, int QM, int RM>
+// LDS region: 8 KiB.  A row's 16-byte pieces are XOR-swizzled by the head, like
+// the K rows: the rotation and the operand reads touch the same piece of 16 rows
+// at once, which unswizzled rows (256 B apart) serialised 16-fold on one group of
+// banks -- 4.5-6 us of every piece for the eight waves together, 1.6-2.5 with the swizzle.
+// Key split: the KS waves of the same tokens share one region, each staging and
+// rotating the heads [kg * 16 / KS, + 16 / KS); read_q_tiles follows a barrier.
+template <int DT, int QM, int RM, int KS>
 __device__ inline void stage_q_tiles(const DecodeParams& p, unsigned char* qreg, float* csreg, const Grp& gr,
-                                     int tok0, int ntile, int f, int hkv, u32x4 (&qB)[kTiles][4]) {
+                                     int tok0, int ntile, int kg, int f, int hkv) {
 #pragma clang fp contract(off)
     using raw = typename Tr<DT>::raw;
     const int lane = opaque_tid() & 63;
-    const int g = lane >> 4, n = lane & 15;
     const uint32_t qbase = lds_addr(qreg);
+    const int half = p.R >> 1;
+    // every load is issued before the first is waited for: cos/sin of both tiles
+    // on clamped, in-bounds indices (a branch around a load waits for it at once)
+    float cv[kTiles], sv[kTiles];
+    const bool rot = QM != kQPre && half > 0;
+    if (rot && ntile > 0) {
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) {
+            const long long row = (long long)f * tok_axis<RM>(p) + gr.lin + tok0 + (t < ntile ? t : 0);
+            const long long co = (QM == kQRotHalf ? row * half : row * p.R) + (lane < half ? lane : 0);
+            cv[t] = p.cosv[co];
+            sv[t] = p.sinv[co];
+        }
+    }
     for (int t = 0; t < ntile; ++t) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i4 = 0; i4 < 4 / KS; ++i4) {
+            const int i = kg * (4 / KS) + i4;
             const int hn = i * 4 + (lane >> 4);
             const int h = hkv * kGqa + hn;
             const raw* q = reinterpret_cast<const raw*>(p.q) + q_row<QM, RM>(p, gr, tok0 + t, h, f);
-            dma16(q + (lane & 15) * 8, __builtin_amdgcn_readfirstlane(qbase + (uint32_t)(t * 4096 + i * 1024)));
+            dma16(q + ((lane & 15) ^ hn) * 8, __builtin_amdgcn_readfirstlane(qbase + (uint32_t)(t * 4096 + i * 1024)));
         }
     }
-    const int half = p.R >> 1;
-    if (QM != kQPre) {
-        for (int t = 0; t < ntile; ++t) {
-            const long long row = (long long)f * tok_axis<RM>(p) + gr.lin + tok0 + t;
-            const long long co = QM == kQRotHalf ? row * half : row * p.R;
-            csreg[t * 128 + lane] = lane < half ? p.cosv[co + lane] : 0.0f;
-            csreg[t * 128 + 64 + lane] = lane < half ? p.sinv[co + lane] : 0.0f;
+    if (rot && ntile > 0) {
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) {
+            csreg[t * 128 + lane] = cv[t];
+            csreg[t * 128 + 64 + lane] = sv[t];
         }
     }
     wait_vmcnt<0>();
     compiler_fence();
-    if (QM != kQPre && half > 0) {
-        const int hn = lane >> 2, q4 = lane & 3;
+    if (rot) {
+        constexpr int kLanes = 4 * KS;  // lanes per head
+        const int hn = kg * (kGqa / KS) + lane / kLanes, q = lane % kLanes;
         for (int t = 0; t < ntile; ++t) {
             raw* x = reinterpret_cast<raw*>(qreg + t * 4096 + hn * 256);
+            auto at = [&](int e) { return x + ((e ^ (hn << 3)) & 127); };  // element e of the row
             const float* cs = csreg + t * 128;
             const float* sn = cs + 64;
             if ((half & 7) == 0) {
-                for (int j0 = q4 * 8; j0 < half; j0 += 32) {
-                    const u32x4 a = *reinterpret_cast<const u32x4*>(x + j0);
-                    const u32x4 b = *reinterpret_cast<const u32x4*>(x + j0 + half);
+                for (int j0 = q * 8; j0 < half; j0 += 8 * kLanes) {
+                    u32x4* pa4 = reinterpret_cast<u32x4*>(at(j0));
+                    u32x4* pb4 = reinterpret_cast<u32x4*>(at(j0 + half));
+                    const u32x4 a = *pa4, b = *pb4;
                     u32x4 ya, yb;
 #pragma unroll
                     for (int e2 = 0; e2 < 4; ++e2) {
-                        uint32_t pa = 0, pb = 0;
+                        uint32_t wa = 0, wb = 0;
 #pragma unroll
                         for (int hl = 0; hl < 2; ++hl) {
                             const int e = e2 * 2 + hl;
                             const float x1 = Tr<DT>::tof((raw)((a[e2] >> (16 * hl)) & 0xffffu));
                             const float x2 = Tr<DT>::tof((raw)((b[e2] >> (16 * hl)) & 0xffffu));
-                            const float c = cs[j0 + e], sv = sn[j0 + e];
-                            const float a1 = x1 * c, b1 = x2 * sv;
-                            const float a2 = x2 * c, b2 = x1 * sv;
-                            pa |= (uint32_t)Tr<DT>::fromf(a1 - b1) << (16 * hl);
-                            pb |= (uint32_t)Tr<DT>::fromf(a2 + b2) << (16 * hl);
+                            const float c = cs[j0 + e], s = sn[j0 + e];
+                            const float a1 = x1 * c, b1 = x2 * s;
+                            const float a2 = x2 * c, b2 = x1 * s;
+                            wa |= (uint32_t)Tr<DT>::fromf(a1 - b1) << (16 * hl);
+                            wb |= (uint32_t)Tr<DT>::fromf(a2 + b2) << (16 * hl);
                         }
-                        ya[e2] = pa;
-                        yb[e2] = pb;
+                        ya[e2] = wa;
+                        yb[e2] = wb;
                     }
-                    *reinterpret_cast<u32x4*>(x + j0) = ya;
-                    *reinterpret_cast<u32x4*>(x + j0 + half) = yb;
+                    *pa4 = ya;
+                    *pb4 = yb;
                 }
             } else {
-                for (int j = q4; j < half; j += 4) {
-                    const float x1 = Tr<DT>::tof(x[j]), x2 = Tr<DT>::tof(x[j + half]);
-                    const float c = cs[j], sv = sn[j];
-                    const float a1 = x1 * c, b1 = x2 * sv;
-                    const float a2 = x2 * c, b2 = x1 * sv;
-                    x[j] = Tr<DT>::fromf(a1 - b1);
-                    x[j + half] = Tr<DT>::fromf(a2 + b2);
+                for (int j = q; j < half; j += kLanes) {
+                    raw *xa = at(j), *xb = at(j + half);
+                    const float x1 = Tr<DT>::tof(*xa), x2 = Tr<DT>::tof(*xb);
+                    const float c = cs[j], s = sn[j];
+                    const float a1 = x1 * c, b1 = x2 * s;
+                    const float a2 = x2 * c, b2 = x1 * s;
+                    *xa = Tr<DT>::fromf(a1 - b1);
+                    *xb = Tr<DT>::fromf(a2 + b2);
                 }
             }
         }
         compiler_fence();
     }
+}
+
+__device__ inline void read_q_tiles(const unsigned char* qreg, int ntile, u32x4 (&qB)[kTiles][4]) {
+    const int lane = opaque_tid() & 63;
+    const int g = lane >> 4, n = lane & 15;
 #pragma unroll
     for (int t = 0; t < kTiles; ++t)
         if (t < ntile)
 #pragma unroll
             for (int cc = 0; cc < 4; ++cc)
-                qB[t][cc] = *reinterpret_cast<const u32x4*>(qreg + t * 4096 + n * 256 + (cc * 32 + g * 8) * 2);
+                qB[t][cc] = *reinterpret_cast<const u32x4*>(qreg + t * 4096 + n * 256 + (((cc * 4 + g) ^ n) << 4));
     compiler_fence();
 }
 
@@ -520,11 +546,15 @@ __device__ inline void combine_split(unsigned char* smem, int wv, int kg, int nt
 // One workgroup: keys [v0, v1) of row group rg for KV head hkv.
 template <int DT, int QM, int KVM, bool P2, int RM, int KS>
 __device__ void chunk_piece(const DecodeParams& p, unsigned char* smem, int* pages, int rg, int hkv, long long v0,
-                            long long v1, bool final_out, int slot) {
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const Grp gr = group_of<RM>(p, rg);
+                            long long v1, bool final_out, int slot, long long row_keys) {
+    const int wv = uniform((int)(threadIdx.x >> 6));
+    Grp gr = group_of<RM>(p, rg);
+    gr.w = uniform(gr.w);
+    gr.s0 = uniform(gr.s0);
+    gr.lin = uniform(gr.lin);
+    gr.ntok = uniform(gr.ntok);
     const int w = gr.w;
-    const int kg = KS == 1 ? 0 : wv / (kWaves / KS);  // this wave's key subset
+    const int kg = KS == 1 ? 0 : wv / (kWaves / KS);                // this wave's key subset
     const int tok0 = (KS == 1 ? wv : wv % (kWaves / KS)) * kTiles;  // and first token of the group
     const int ntile = gr.ntok - tok0 < kTiles ? (gr.ntok - tok0 > 0 ? gr.ntok - tok0 : 0) : kTiles;
 
@@ -540,21 +570,21 @@ __device__ void chunk_piece(const DecodeParams& p, unsigned char* smem, int* pag
 
     long long P = 0, off = 0;
     for (int f = 0; f < p.F && P < v1; ++f) {
-        // visible keys of this view for the block (union) and per tile
-        const int vis_blk = group_view_vis<KVM, RM>(p, f, gr);
+        // visible keys per tile (wave-uniform: the stage masks and their branches
+        // stay scalar), and of this view for the block: the union over its tokens,
+        // for a single view the row's keys, counted by the schedule
         int vis_t[kTiles];
 #pragma unroll
-        for (int t = 0; t < kTiles; ++t)  // wave-uniform: the stage masks and their branches stay scalar
-            vis_t[t] = __builtin_amdgcn_readfirstlane(t < ntile ? view_vis<KVM>(p, f, loc_of<RM>(p, f, gr, tok0 + t)) : 0);
+        for (int t = 0; t < kTiles; ++t) {
+            const int last = gr.ntok - 1;  // >= 0: a group without tokens has no piece
+            const int v = uniform(view_vis<KVM>(p, f, loc_of<RM>(p, f, gr, tok0 + t < last ? tok0 + t : last)));
+            vis_t[t] = t < ntile ? v : 0;
+        }
+        const int vis_blk = p.F == 1 ? (int)row_keys : uniform(group_view_vis<KVM, RM>(p, f, gr));
         const long long a = v0 > P ? v0 : P;
         const long long bnd = v1 < P + vis_blk ? v1 : P + vis_blk;
         if (a < bnd) {
-            u32x4 qB[kTiles][4] = {};
-            // the ring is idle here (previous range drained): stage the query tiles in it
-            stage_q_tiles<DT, QM, RM>(p, smem + wv * (kTiles * 4096),
-                                      reinterpret_cast<float*>(smem + kWaves * kTiles * 4096 + wv * kTiles * 512), gr,
-                                      tok0, ntile, f, hkv, qB);
-            __syncthreads();
+            const int la = (int)(a - P), lb = (int)(bnd - P);
             Range r;
             r.w = w;
             r.hkv = hkv;
@@ -572,22 +602,39 @@ __device__ void chunk_piece(const DecodeParams& p, unsigned char* smem, int* pag
                 r.bstride = fd.bstride * w;
                 r.L = fd.L;
             }
-            const int la = (int)(a - P), lb = (int)(bnd - P);
+            u32x4 qB[kTiles][4] = {};
             // sub-ranges whose page ids fit the LDS page cache
             const int span = KVM == kKvPaged ? (p.bs_shift >= 0 ? (kPageCap - 2) << p.bs_shift : (kPageCap - 2) * p.bs)
                                              : (1 << 30);
             for (int sa = la; sa < lb; sa += span) {
                 const int sbnd = sa + span < lb ? sa + span : lb;
                 r.b = sbnd;
-                r.pages_ok = true;
+                int pg[kPageIt];
+                uint32_t lpl = 0;
+                r.lp0 = 0;
                 if (KVM == kKvPaged) {
                     const uint32_t p0 = (uint32_t)(off + sa), p1 = (uint32_t)(off + sbnd - 1);
-                    const uint32_t lpl = p.bs_shift >= 0 ? (p1 >> p.bs_shift) : p1 / (uint32_t)p.bs;
+                    lpl = p.bs_shift >= 0 ? (p1 >> p.bs_shift) : p1 / (uint32_t)p.bs;
                     r.lp0 = p.bs_shift >= 0 ? (p0 >> p.bs_shift) : p0 / (uint32_t)p.bs;
+                    fetch_pages(p, p.bt + (long long)w * p.maxB, r.lp0, lpl, pg);
+                }
+                // the ring is idle here (previous range drained): stage the query tiles
+                // in it, their round trip beside the page ids'
+                unsigned char* qreg = smem + (KS == 1 ? wv : wv % (kWaves / KS)) * (kTiles * 4096);
+                if (sa == la) {
+                    stage_q_tiles<DT, QM, RM, KS>(
+                        p, qreg, reinterpret_cast<float*>(smem + kWaves * kTiles * 4096 + wv * kTiles * 512), gr, tok0,
+                        ntile, kg, f, hkv);
+                    if (KS == 1) read_q_tiles(qreg, ntile, qB);
+                }
+                // every page of the sub-range is valid; the page ids are written and the
+                // query tiles read (KS > 1: staged)
+                bool ok = true;
+                if (KVM == kKvPaged) ok = store_pages(p, pages, r.lp0, lpl, pg);
+                r.pages_ok = __syncthreads_and(ok) != 0;
+                if (KS > 1 && sa == la) {
+                    read_q_tiles(qreg, ntile, qB);
                     __syncthreads();
-                    // every page this thread loaded for the sub-range is valid
-                    const bool ok = fill_page_cache(p, p.bt + (long long)w * p.maxB, pages, r.lp0, lpl);
-                    r.pages_ok = __syncthreads_and(ok) != 0;
                 }
                 stream_range<DT, KVM, P2, KS>(p, r, pages, smem, sa, sbnd, kg, vis_t, qB, tl);
             }
@@ -640,8 +687,10 @@ __global__ __launch_bounds__(kThreads) void dv_chunk(const DecodeParams p) {
     const int NHG = p.Hkv;  // one KV head per workgroup
 
     run_schedule(p, NHG, s_pref, s_scan, [&](int rg) { return group_visible<KVM, RM>(p, rg); },
-                 [&](int rg, int hg, long long v0, long long v1, bool fin, int slot, long long) {
-                     chunk_piece<DT, QM, KVM, P2, RM, KS>(p, smem, pages, rg, hg, v0, v1, fin, slot);
+                 [&](int rg, int hg, long long v0, long long v1, bool fin, int slot, long long rk) {
+                     chunk_piece<DT, QM, KVM, P2, RM, KS>(p, smem, pages, uniform(rg), uniform(hg), uniform(v0),
+                                                          uniform(v1), uniform((int)fin) != 0, uniform(slot),
+                                                          uniform(rk));
                  });
 }
 
@@ -657,11 +706,13 @@ size_t lds_bytes(int nrows) {
 // maximum of cu_seqlens_q[1 .. i + 1], sequence i's tokens are therefore
 // [max(0, M_{i-1}), min(T, M_i)) (M_{-1} = 0), and the tokens from M_{W-1} on
 // form one more run, of sequence 0 -- also for tables that are not
-// non-decreasing.  Each run is cut into groups of kTokBlk tokens.  One
-// workgroup writes entry g = {first token, tokens, sequence, 0} for every
-// group, and {0, 0, 0, 0} for the entries from the group count up to gmax
-// (the host's bound T / kTokBlk + W + 1: a run of n tokens makes at most
-// n / kTokBlk + 1 groups).
+// non-decreasing.  Each run is cut into groups of kTokBlk tokens; a last group of
+// at most `few` tokens goes to a list of its own, for a launch that splits the
+// keys (batches of decodes and prompt chunks: a decode's group would otherwise
+// be computed as 16 tokens).  One workgroup writes entry g = {first token,
+// tokens, sequence, 0} of every group of the two lists -- gmax entries for the
+// first, then W + 1 for the short groups (few > 0) -- and {0, 0, 0, 0} past each
+// list's end.  gmax is the host's bound (varlen_gmax).
 constexpr int kVgThreads = 1024;
 
 __device__ inline int block_scan_excl(int v, int* s_part, bool is_max) {
@@ -683,9 +734,10 @@ __device__ inline int block_scan_excl(int v, int* s_part, bool is_max) {
     return is_max ? (mine > before ? mine : before) : before + mine;
 }
 
-__global__ __launch_bounds__(kVgThreads) void dv_varlen_groups(const int* cu, int W, int T, int gmax, int4* groups) {
+__global__ __launch_bounds__(kVgThreads) void dv_varlen_groups(const int* cu, int W, int T, int few, int gmax, int4* groups) {
     __shared__ int s_m[kVarlenChunkMaxW];       // M_i
-    __shared__ int s_base[kVarlenChunkMaxW + 2];  // first group of run i (runs 0 .. W), then the total
+    __shared__ int s_base[kVarlenChunkMaxW + 2];   // first group of run i (runs 0 .. W), then the total
+    __shared__ int s_sbase[kVarlenChunkMaxW + 2];  // the same for the short groups
     __shared__ int s_part[kVgThreads / kWave];
     const int tid = threadIdx.x;
     // running maximum of cu[1 .. W], each thread over a contiguous block of sequences
@@ -707,41 +759,60 @@ __global__ __launch_bounds__(kVgThreads) void dv_varlen_groups(const int* cu, in
     };
     const int per1 = (W + 1 + kVgThreads - 1) / kVgThreads;
     const int j0 = tid * per1 < W + 1 ? tid * per1 : W + 1, j1 = j0 + per1 < W + 1 ? j0 + per1 : W + 1;
-    int cnt = 0;
-    for (int i = j0; i < j1; ++i) {
+    // groups of a run: {full or long ones, short ones}
+    auto count = [&](int i, int& c, int& sc) {
         int a, b;
         run(i, a, b);
-        const int c = b > a ? (b - a + kTokBlk - 1) / kTokBlk : 0;
-        s_base[i] = c;
+        const int n = b > a ? b - a : 0, rem = n % kTokBlk;
+        sc = rem > 0 && rem <= few ? 1 : 0;
+        c = n / kTokBlk + (rem > few ? 1 : 0);
+    };
+    int cnt = 0, scnt = 0;
+    for (int i = j0; i < j1; ++i) {
+        int c, sc;
+        count(i, c, sc);
         cnt += c;
+        scnt += sc;
     }
     int acc = block_scan_excl(cnt, s_part, false);
-    for (int i = j0; i < j1; ++i) {
-        const int c = s_base[i];
-        s_base[i] = acc;
-        acc += c;
-    }
-    if (tid == kVgThreads - 1) s_base[W + 1] = acc;
     __syncthreads();
-    const int total = s_base[W + 1];
-    for (int gi = tid; gi < gmax; gi += kVgThreads) {
+    int sacc = block_scan_excl(scnt, s_part, false);
+    for (int i = j0; i < j1; ++i) {
+        int c, sc;
+        count(i, c, sc);
+        s_base[i] = acc;
+        s_sbase[i] = sacc;
+        acc += c;
+        sacc += sc;
+    }
+    if (tid == kVgThreads - 1) {
+        s_base[W + 1] = acc;
+        s_sbase[W + 1] = sacc;
+    }
+    __syncthreads();
+    const int total = s_base[W + 1], stotal = s_sbase[W + 1];
+    const int entries = gmax + (few > 0 ? W + 1 : 0);
+    for (int e0 = tid; e0 < entries; e0 += kVgThreads) {
         int4 e = {0, 0, 0, 0};
-        if (gi < total) {
+        const bool is_short = e0 >= gmax;
+        const int gi = is_short ? e0 - gmax : e0;
+        const int* base = is_short ? s_sbase : s_base;
+        if (gi < (is_short ? stotal : total)) {
             // the last run whose first group is <= gi (it has groups: the next run's first is larger)
             int lo = 0, hi = W;
             while (lo < hi) {
                 const int mid = (lo + hi + 1) >> 1;
-                if (s_base[mid] <= gi) lo = mid;
+                if (base[mid] <= gi) lo = mid;
                 else hi = mid - 1;
             }
             int a, b;
             run(lo, a, b);
-            const int t0 = a + (gi - s_base[lo]) * kTokBlk;
+            const int t0 = a + (is_short ? (b - a) / kTokBlk : gi - base[lo]) * kTokBlk;
             e.x = t0;
             e.y = b - t0 < kTokBlk ? b - t0 : kTokBlk;
             e.z = lo == W ? 0 : lo;
         }
-        groups[gi] = e;
+        groups[e0] = e;
     }
 }
 
@@ -760,7 +831,8 @@ hipError_t launch1(DecodeParams p, int device, int cus, long long cap, hipStream
     hipLaunchKernelGGL((dv_chunk<DT, QM, KVM, P2, RM, KS>), dim3(p.nwg), dim3(kThreads), lds, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const int ntb = max_group_tokens<RM>(p);
+    int ntb = max_group_tokens<RM>(p);
+    if (KS == 4 && ntb > kFewTok) ntb = kFewTok;
     hipLaunchKernelGGL((dv_merge_chunk<DT, RM>), dim3(p.nrows * p.Hkv * ntb), dim3(256), 0, stream, p, ntb);
     return hipGetLastError();
 }
@@ -768,7 +840,8 @@ hipError_t launch1(DecodeParams p, int device, int cus, long long cap, hipStream
 template <int DT, int QM, int KVM, int RM, bool P2>
 hipError_t launch_split(const DecodeParams& p, int ks, int device, int cus, long long cap, hipStream_t stream) {
     if (ks == 4) return launch1<DT, QM, KVM, P2, RM, 4>(p, device, cus, cap, stream);
-    if (ks == 2) return launch1<DT, QM, KVM, P2, RM, 2>(p, device, cus, cap, stream);
+    if constexpr (RM != kRowVarlen)  // varlen launches: groups of at most kFewTok tokens, or any
+        if (ks == 2) return launch1<DT, QM, KVM, P2, RM, 2>(p, device, cus, cap, stream);
     return launch1<DT, QM, KVM, P2, RM, 1>(p, device, cus, cap, stream);
 }
 
@@ -790,7 +863,7 @@ hipError_t launch(const DecodeParams& p, int ks, int device, int cus, long long 
 // softmax, which -inf scores only do for a positive scale.
 int key_split(float l2scale, int ntok) {
     if (!(l2scale > 0.0f) || ntok > 8) return 1;
-    return ntok > 4 ? 2 : 4;
+    return ntok > kFewTok ? 2 : 4;
 }
 
 }  // namespace chunk
@@ -811,17 +884,25 @@ ChunkWs chunk_ws(long long groups, int Hkv, int device, bool varlen) {
     ChunkWs l;
     l.part = ((size_t)((chunk_cus(device) + nseg) * slot_floats * 4) + 255) & ~(size_t)255;
     l.dir = ((size_t)(nseg * 2 * 4) + 255) & ~(size_t)255;
-    l.vgroups = varlen ? (size_t)groups * 16 : 0;
+    l.vgroups = varlen ? (size_t)groups * 2 * 16 : 0;  // two lists (dv_varlen_groups)
     l.total = l.part + l.dir + l.vgroups;
     return l;
 }
 
-long long varlen_gmax(int T, int W) { return (long long)T / chunk::kTokBlk + W + 1; }
+// Groups of a varlen call at most: a run of n tokens makes n / kTokBlk of
+// kTokBlk tokens and one more, and there are W + 1 runs; with short groups listed
+// apart, the others have more than kFewTok tokens.
+long long varlen_gmax(int T, int W, bool few) {
+    const long long g = (long long)T / chunk::kTokBlk + W + 1;
+    const long long n = T / (chunk::kFewTok + 1);
+    return few && n < g ? n : g;
+}
 
 // The chunk launches over `groups` row groups, kMaxRows at a time.
 template <int RM>
 hipError_t launch_groups(int dtype, int qmode, int kvmode, DecodeParams p, long long groups_total,
-                         long long max_keys_per_group, const ChunkWs& l, void* workspace, hipStream_t stream) {
+                         long long max_keys_per_group, int ks, const ChunkWs& l, void* workspace,
+                         hipStream_t stream) {
     int device = 0;
     hipError_t e = hipGetDevice(&device);
     if (e != hipSuccess) return e;
@@ -830,7 +911,6 @@ hipError_t launch_groups(int dtype, int qmode, int kvmode, DecodeParams p, long 
     p.slot_floats = chunk::kTokBlk * kGqa * (kHeadDim + 1);
     p.part = reinterpret_cast<float*>(workspace);
     p.dir = reinterpret_cast<int*>(reinterpret_cast<unsigned char*>(workspace) + l.part);
-    const int ks = RM == kRowVarlen || dtype == kF32 ? 1 : chunk::key_split(p.l2scale, p.S);
     p.piece_cost = ks == 1 ? chunk::kPieceCost : chunk::kPieceCostSplit;
     // odd workgroups (odd XCD of each pair) take shorter chunks, as in the decode
     // split; 30 per mille measured best on configuration 5
@@ -886,12 +966,13 @@ hipError_t launch_chunk(int dtype, int qmode, int kvmode, const DecodeParams& ba
     const long long groups = (long long)base.W * ((base.S + chunk::kTokBlk - 1) / chunk::kTokBlk);
     const ChunkWs l = chunk_ws(groups, base.Hkv, device, false);
     if (ws_bytes < l.total) return hipErrorInvalidValue;
-    return launch_groups<kRowWS>(dtype, qmode, kvmode, base, groups, max_keys_per_group, l, workspace, stream);
+    const int ks = dtype == kF32 ? 1 : chunk::key_split(base.l2scale, base.S);
+    return launch_groups<kRowWS>(dtype, qmode, kvmode, base, groups, max_keys_per_group, ks, l, workspace, stream);
 }
 
 size_t varlen_chunk_workspace_bytes(int T, int W, int Hkv, int device) {
     if (T <= 0 || W <= 0 || Hkv <= 0) return 0;
-    return chunk_ws(varlen_gmax(T, W), Hkv, device, true).total;
+    return chunk_ws(varlen_gmax(T, W, false), Hkv, device, true).total;
 }
 
 hipError_t launch_varlen_chunk(int dtype, const DecodeParams& base, long long max_keys_per_group, void* workspace,
@@ -901,17 +982,28 @@ hipError_t launch_varlen_chunk(int dtype, const DecodeParams& base, long long ma
     int device = 0;
     hipError_t e = hipGetDevice(&device);
     if (e != hipSuccess) return e;
-    const long long gmax = varlen_gmax(base.T, base.W);
-    const ChunkWs l = chunk_ws(gmax, base.Hkv, device, true);
+    const ChunkWs l = chunk_ws(varlen_gmax(base.T, base.W, false), base.Hkv, device, true);
     if (ws_bytes < l.total) return hipErrorInvalidValue;
+    // the decodes of a mixed batch apart from its chunks (16-bit types; a key
+    // split needs a positive scale)
+    const int ks = dtype == kF32 ? 1 : chunk::key_split(base.l2scale, chunk::kFewTok);
+    const int few = ks > 1 ? chunk::kFewTok : 0;
+    const long long gmax = varlen_gmax(base.T, base.W, few > 0);
     DecodeParams p = base;
     int4* groups = reinterpret_cast<int4*>(reinterpret_cast<unsigned char*>(workspace) + l.part + l.dir);
-    p.vgroups = reinterpret_cast<const int*>(groups);
     hipLaunchKernelGGL(chunk::dv_varlen_groups, dim3(1), dim3(chunk::kVgThreads), 0, stream, base.cu_q, base.W,
-                       base.T, (int)gmax, groups);
+                       base.T, few, (int)gmax, groups);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return launch_groups<kRowVarlen>(dtype, kQRotHalf, kKvPaged, p, gmax, max_keys_per_group, l, workspace, stream);
+    // one launch after the other on the same partial slots
+    if (few > 0) {
+        p.vgroups = reinterpret_cast<const int*>(groups + gmax);
+        e = launch_groups<kRowVarlen>(dtype, kQRotHalf, kKvPaged, p, base.W + 1, max_keys_per_group, ks, l, workspace,
+                                      stream);
+        if (e != hipSuccess || gmax == 0) return e;
+    }
+    p.vgroups = reinterpret_cast<const int*>(groups);
+    return launch_groups<kRowVarlen>(dtype, kQRotHalf, kKvPaged, p, gmax, max_keys_per_group, 1, l, workspace, stream);
 }
 
 }  // namespace dv

@@ -263,7 +263,11 @@ __device__ void chunk32_piece(const DecodeParams& p, unsigned char* smem, int* p
                     r.lp0 = p.bs_shift >= 0 ? (p0 >> p.bs_shift) : p0 / (uint32_t)p.bs;
                     __syncthreads();  // every wave is done with the previous sub-range's page ids
                     static_assert(kWaves32 * kWave == kThreads, "one page-cache fill per workgroup");
-                    fill_page_cache(p, p.bt + (long long)w * p.maxB, pages, r.lp0, 0u);
+                    const uint32_t p1 = (uint32_t)(off + sbnd - 1);
+                    const uint32_t lpl = p.bs_shift >= 0 ? (p1 >> p.bs_shift) : p1 / (uint32_t)p.bs;
+                    int pg[kPageIt];
+                    fetch_pages(p, p.bt + (long long)w * p.maxB, r.lp0, lpl, pg);
+                    store_pages(p, pages, r.lp0, lpl, pg);
                     __syncthreads();
                 }
                 stream32<KVM, P2>(p, r, pages, smem, sa, sbnd, nt, vis_t, qB, tl);

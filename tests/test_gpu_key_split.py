@@ -3,13 +3,14 @@ oracle: row groups whose keys are split over the waves of a workgroup (two or
 four wave sets, dvattention_amd/csrc/dv_chunk.hip) and the first size past it.
 Lengths end inside the first stage, the first step of a split and a later one,
 so some wave sets see no key; ragged batches also leave pieces of a few keys to
-merge.  Tolerances: test_gpu_parity.close."""
+merge.  Packed batches mix short row groups with long ones.  Tolerances:
+test_gpu_parity.close."""
 import numpy as np
 import pytest
 import torch
 
 from oracle import dvattn_oracle as O
-from test_gpu_parity import close, dv, rand_paged, run_paged  # noqa: F401
+from test_gpu_parity import close, dv, rand_paged, rand_varlen, run_paged, run_varlen  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +38,20 @@ def test_contiguous_few_tokens(dv, gpu, S):  # noqa: F811
     fl = torch.tensor(Ls, dtype=torch.int32)
     out = dv.dvattn_sdpa(q.to(gpu), loc.to(gpu), [k.to(gpu) for k in ks], [v.to(gpu) for v in vs], 0.1, fl.to(gpu))
     close(out, O.contig_sdpa(0.1, loc, q, fl, ks, vs), torch.bfloat16, f"S={S}")
+
+
+# tokens per sequence: groups of 4 or fewer are listed apart from longer ones
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("counts,lens", [
+    ([1, 1, 40, 1, 3], [700]), ([4, 5, 16, 17, 20, 21, 0, 1], [90, 40]), ([2, 2], [50]), ([16, 32], [300]),
+    ([1] * 6 + [30], [2000, 33, 0])])
+def test_varlen_mixed_groups(dv, gpu, dtype, counts, lens):  # noqa: F811
+    W, T = len(counts), sum(counts)
+    d = rand_varlen(len(lens), W, T, np.concatenate([[0], np.cumsum(counts)]), 2, 16, lens, 64, dtype, seed=T)
+    close(run_varlen(dv, d, 0.1, gpu), O.varlen_paged_sdpa(0.1, **d), dtype, f"{counts}")
+
+
+def test_varlen_mixed_unsorted_table(dv, gpu):  # noqa: F811
+    # a table that is not non-decreasing, and tokens past its last entry
+    d = rand_varlen(2, 4, 45, np.array([0, 3, 2, 30, 29]), 1, 16, [60, 200], 32, torch.bfloat16, seed=5)
+    close(run_varlen(dv, d, 0.1, gpu), O.varlen_paged_sdpa(0.1, **d), torch.bfloat16, "unsorted")
