@@ -686,6 +686,8 @@ __global__ __launch_bounds__(kThreads) void dv_chunk(const DecodeParams p) {
     long long* s_pref = s_scan + kWaves;
     const int NHG = p.Hkv;  // one KV head per workgroup
 
+    // an empty list of groups (varlen): no cost to lay out, no piece
+    if (RM == kRowVarlen && blockIdx.x > 0 && p.vgroups[p.row_begin * 4 + 1] == 0) return;
     run_schedule(p, NHG, s_pref, s_scan, [&](int rg) { return group_visible<KVM, RM>(p, rg); },
                  [&](int rg, int hg, long long v0, long long v1, bool fin, int slot, long long rk) {
                      chunk_piece<DT, QM, KVM, P2, RM, KS>(p, smem, pages, uniform(rg), uniform(hg), uniform(v0),
@@ -898,6 +900,10 @@ long long varlen_gmax(int T, int W, bool few) {
     return few && n < g ? n : g;
 }
 
+// Keys (of all sequences and KV heads) from which a varlen call lists its short
+// groups apart.
+constexpr long long kFewMinKeys = 1ll << 18;
+
 // The chunk launches over `groups` row groups, kMaxRows at a time.
 template <int RM>
 hipError_t launch_groups(int dtype, int qmode, int kvmode, DecodeParams p, long long groups_total,
@@ -985,8 +991,14 @@ hipError_t launch_varlen_chunk(int dtype, const DecodeParams& base, long long ma
     const ChunkWs l = chunk_ws(varlen_gmax(base.T, base.W, false), base.Hkv, device, true);
     if (ws_bytes < l.total) return hipErrorInvalidValue;
     // the decodes of a mixed batch apart from its chunks (16-bit types; a key
-    // split needs a positive scale)
-    const int ks = dtype == kF32 ? 1 : chunk::key_split(base.l2scale, chunk::kFewTok);
+    // split needs a positive scale), where the sequences' keys are worth the
+    // second launch and merge: those cost 5 us of a call without short groups
+    // (2 x 64 tokens, 500 keys, 8 KV heads: 43.5 -> 48.3 us; 4 x 4 x 500: 31.4 ->
+    // 36.8), the split saves a quarter of a call of short ones (32 x 4 x 4608
+    // keys: 185 -> 124 us)
+    const int ks = dtype == kF32 || base.W * (long long)base.Hkv * max_keys_per_group < kFewMinKeys
+                       ? 1
+                       : chunk::key_split(base.l2scale, chunk::kFewTok);
     const int few = ks > 1 ? chunk::kFewTok : 0;
     const long long gmax = varlen_gmax(base.T, base.W, few > 0);
     DecodeParams p = base;
