@@ -188,16 +188,26 @@ __global__ __launch_bounds__(256) void dv_view_meta(const MetaParams p, long lon
     const int w = (int)(fw % p.W);
     const int f = (int)(fw / p.W);
     // the whole row is walked: if f appears more than once, its first place
-    // wins, as in the reference, whose backward walk assigns it last
+    // wins, as in the reference, whose backward walk assigns it last.  The row is
+    // walked eight segments at a time, their loads issued together (one after the
+    // other, a row of five segments was ten dependent round trips)
     long long suffix = 0, at = 0;
     bool found = false;
     const int* ord = p.order + (long long)w * p.F;
-    for (int j = p.F - 1; j >= 0; --j) {
-        const int g = ord[j];
-        if (g >= 0 && g < p.F) suffix += p.fl[g];
-        if (g == f) {
-            found = true;
-            at = suffix;
+    for (int j0 = p.F - 1; j0 >= 0; j0 -= 8) {
+        int g[8], len[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) g[k] = ord[j0 - k > 0 ? j0 - k : 0];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) len[k] = p.fl[g[k] >= 0 && g[k] < p.F ? g[k] : 0];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            if (j0 - k < 0) continue;
+            if (g[k] >= 0 && g[k] < p.F) suffix += len[k];
+            if (g[k] == f) {
+                found = true;
+                at = suffix;
+            }
         }
     }
     const int loc = found ? (int)(at - p.S + s) : -1;

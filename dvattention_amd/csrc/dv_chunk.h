@@ -208,15 +208,6 @@ __device__ inline bool store_pages(const DecodeParams& p, int* pages, uint32_t l
     return ok;
 }
 
-// A wave-uniform value computed per lane, moved to scalar registers.
-__device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ inline long long uniform(long long v) {
-    const unsigned long long u = (unsigned long long)v;
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
-    return (long long)(((unsigned long long)hi << 32) | lo);
-}
-
 // Tokens of the largest row group of a launch (the token blocks of its merge).
 template <int RM>
 inline int max_group_tokens(const DecodeParams& p) {

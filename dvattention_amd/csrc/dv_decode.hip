@@ -363,7 +363,7 @@ __device__ inline void compute(SoftState& st, const unsigned char* kt, const uns
     if constexpr (DT == kF16)
 #pragma unroll
         for (int cc = 0; cc < 8; ++cc) st.o[cc] = Tr<DT>::mma(vA[cc], pB.lo, st.o[cc]);
-    mfma_settle(st.o);
+    mfma_settle_acc(st.o);
 }
 
 constexpr int kStreamViews = 4;  // views of one piece streamed back to back
@@ -377,10 +377,9 @@ constexpr int kStreamViews = 4;  // views of one piece streamed back to back
 template <int DT, int QM, int RM>
 __device__ bool views_stream(const DecodeParams& p, unsigned char* wlds, int row, int w, int hkv, long long v0,
                              long long v1, uint64_t vm, const ViewTab& t, SoftState& st) {
-    const int lane = threadIdx.x & 63;
     const uint32_t ring = __builtin_amdgcn_readfirstlane(lds_addr(wlds));
     int* pc = reinterpret_cast<int*>(wlds + kRing * kStage);
-    int vf[kStreamViews], l0[kStreamViews], l1[kStreamViews], ns[kStreamViews], pcb[kStreamViews + 1];
+    int vf[kStreamViews], ls[kStreamViews], l0[kStreamViews], l1[kStreamViews], ns[kStreamViews], pcb[kStreamViews + 1];
     int voff[kStreamViews], lpa[kStreamViews];
     int npages = 0, N = 0;
     uint64_t m = vm;
@@ -389,22 +388,23 @@ __device__ bool views_stream(const DecodeParams& p, unsigned char* wlds, int row
         const bool has = m != 0;
         const int f = has ? __builtin_ctzll(m) : 0;
         m &= m - 1;
-        const int vis = __shfl(t.vis, f, kWave);
-        const long long P = __shfl(t.P, f, kWave);
-        const long long off = __shfl(t.off, f, kWave);
+        const int vis = uniform(__shfl(t.vis, f, kWave));
+        const long long P = uniform(__shfl(t.P, f, kWave));
+        const long long off = uniform(__shfl(t.off, f, kWave));
         const long long a = v0 > P ? v0 : P;
         const long long b = v1 < P + vis ? v1 : P + vis;
         vf[j] = f;
         l0[j] = has ? (int)(a - P) : 0;
         l1[j] = has ? (int)(b - P) : 0;
-        ns[j] = (l1[j] - l0[j] + kStep - 1) / kStep;
-        N += ns[j];
         voff[j] = (int)off;
+        ls[j] = has ? stage_start<kKvPaged>(voff[j], l0[j]) : 0;
+        ns[j] = (l1[j] - ls[j] + kStep - 1) / kStep;
+        N += ns[j];
         lpa[j] = 0;
         pcb[j] = npages;
         if (has) {
             uint32_t la, lz, r;
-            const int pa = voff[j] + l0[j], pz = voff[j] + l1[j] - 1;
+            const int pa = voff[j] + ls[j], pz = voff[j] + l1[j] - 1;
             page_split(p, pa > 0 ? (uint32_t)pa : 0u, la, r);
             page_split(p, pz > 0 ? (uint32_t)pz : 0u, lz, r);
             lpa[j] = (int)la;
@@ -445,9 +445,11 @@ __device__ bool views_stream(const DecodeParams& p, unsigned char* wlds, int row
     vi.v = reinterpret_cast<const unsigned char*>(p.vc);
     vi.off = voff[0];
     vi.lp0 = lpa[0];
+    vi.a = l0[0];
     vi.b = l1[0];
+    const LaneOff lo = lane_offsets((uint32_t)p.Hkv << 8);
     const int* pci = pc;
-    int ji = 0, li = l0[0];
+    int ji = 0, li = ls[0];
     auto advance = [&]() {
         li += kStep;
         if (li >= vi.b) {
@@ -457,17 +459,18 @@ __device__ bool views_stream(const DecodeParams& p, unsigned char* wlds, int row
                 if (k == ji) {
                     vi.off = voff[k];
                     vi.lp0 = lpa[k];
+                    vi.a = l0[k];
                     vi.b = l1[k];
                     pci = pc + pcb[k];
-                    li = l0[k];
+                    li = ls[k];
                 }
         }
     };
-    uint32_t m0 = issue<kKvPaged>(p, vi, pci, ring, li);
+    uint32_t m0 = issue_stage(p, vi, lo, pci, ring, li);
     advance();
     uint32_t m1 = 0;
     if (N > 1) {
-        m1 = issue<kKvPaged>(p, vi, pci, ring + kStage, li);
+        m1 = issue_stage(p, vi, lo, pci, ring + kStage, li);
         advance();
     }
     // rotated queries of every view while the first stages are in flight, then
@@ -499,7 +502,7 @@ __device__ bool views_stream(const DecodeParams& p, unsigned char* wlds, int row
         compute<DT>(st, kt, kt + kTile, (s & 1) ? m1 : m0, qc, p.l2scale);
         if (s + 2 < N) {
             lds_wait();  // the slot's reads are complete before it is refilled
-            const uint32_t mk = issue<kKvPaged>(p, vi, pci, ring + (uint32_t)((s & 1) * kStage), li);
+            const uint32_t mk = issue_stage(p, vi, lo, pci, ring + (uint32_t)((s & 1) * kStage), li);
             advance();
             if (s & 1) m1 = mk;
             else m0 = mk;
@@ -567,6 +570,8 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
             const int l0 = (int)(a - P), l1 = (int)(bnd - P);
             View v;
             v.hkv = hkv;
+            v.a = l0;
+            const LaneOff lo = lane_offsets(KVM == kKvPaged ? (uint32_t)p.Hkv << 8 : 256u);
             if (KVM == kKvPaged) {
                 v.k = reinterpret_cast<const unsigned char*>(p.kc);
                 v.v = reinterpret_cast<const unsigned char*>(p.vc);
@@ -574,8 +579,8 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
             } else {
                 const FragDesc& fd = frag<KVM>(p, f);
                 const long long base = (fd.bstride * w + (long long)hkv * fd.L * kHeadDim) * 2;
-                v.k = reinterpret_cast<const unsigned char*>(fd.k) + base;
-                v.v = reinterpret_cast<const unsigned char*>(fd.v) + base;
+                v.k = reinterpret_cast<const unsigned char*>(uniform((long long)(uintptr_t)fd.k + base));
+                v.v = reinterpret_cast<const unsigned char*>(uniform((long long)(uintptr_t)fd.v + base));
                 v.off = 0;
             }
             v.lp0 = 0;
@@ -585,9 +590,13 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
             const bool qsplit = q_split<QM>(p);
             QRaw qr;
             if (qsplit) fetch_q16<DT, QM, RM>(p, row, f, hkv, qr);
-            // sub-ranges whose pages fit the page cache
-            const long long span = KVM == kKvPaged ? (long long)(kPc - 1) * p.bs : (1ll << 30);
-            for (int sa = l0; sa < l1;) {
+            // sub-ranges whose pages fit the page cache, whole stages
+            long long span = 1ll << 30;
+            if (KVM == kKvPaged) {
+                span = ((long long)(kPc - 2) * p.bs) & ~(long long)(kStep - 1);
+                span = span < (1ll << 30) ? span : 1ll << 30;
+            }
+            for (int sa = stage_start<KVM>(v.off, l0); sa < l1;) {
                 const int sb = (long long)l1 - sa > span ? (int)(sa + span) : l1;
                 v.b = sb;
                 if (KVM == kKvPaged) {
@@ -601,9 +610,15 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
                                [&](int i) { return lpa + (uint32_t)i; });
                 }
                 const int n_st = (sb - sa + kStep - 1) / kStep;
-                uint32_t m0 = issue<KVM>(p, v, pc, ring, sa);
-                uint32_t m1 = 0;
-                if (n_st > 1) m1 = issue<KVM>(p, v, pc, ring + kStage, sa + kStep);
+                // the first two stages in a rolled loop: this code runs once per piece,
+                // and a second copy of it would be fetched cold
+                uint32_t m0 = 0, m1 = 0;
+#pragma unroll 1
+                for (int s = 0; s < 2 && s < n_st; ++s) {
+                    m0 = m1;
+                    m1 = issue_keys<KVM>(p, v, lo, pc, ring + (uint32_t)(s * kStage), sa + s * kStep);
+                }
+                if (n_st == 1) m0 = m1;
                 if (!have_q) {
                     // rotated once per (row, view) while the first stages are in flight
                     if (qsplit) rotate_q16<DT, QM>(qr, qB);
@@ -621,7 +636,7 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
                     compute<DT>(st, kt, kt + kTile, (s & 1) ? m1 : m0, qB, p.l2scale);
                     if (s + 2 < n_st) {
                         lds_wait();  // the slot's reads are complete before it is refilled
-                        const uint32_t mk = issue<KVM>(p, v, pc, ring + (uint32_t)((s & 1) * kStage),
+                        const uint32_t mk = issue_keys<KVM>(p, v, lo, pc, ring + (uint32_t)((s & 1) * kStage),
                                                        sa + (s + 2) * kStep);
                         if (s & 1) m1 = mk;
                         else m0 = mk;
@@ -633,7 +648,7 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
         }
     };
     if (p.F <= kWave) {
-        uint64_t vm = ballot(lane < p.F && t.vis > 0 && t.P < v1 && t.P + t.vis > v0);
+        uint64_t vm = v0 < v1 ? ballot(lane < p.F && t.vis > 0 && t.P < v1 && t.P + t.vis > v0) : 0;
         const int nv = __builtin_popcountll(vm);
         bool done = false;
         if constexpr (MV && KVM == kKvPaged) {
@@ -642,10 +657,13 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
         while (!done && vm) {
             const int f = __builtin_ctzll(vm);
             vm &= vm - 1;
-            one_view(f, __shfl(t.vis, f, kWave), __shfl(t.P, f, kWave), __shfl(t.off, f, kWave));
+            one_view(f, uniform(__shfl(t.vis, f, kWave)), uniform(__shfl(t.P, f, kWave)),
+                     uniform(__shfl(t.off, f, kWave)));
         }
-    } else {
-        for_views<KVM, RM>(p, row, v0, v1, one_view);
+    } else if (v0 < v1) {
+        for_views<KVM, RM>(p, row, v0, v1, [&](int f, int vis, long long P, long long off) {
+            one_view(f, uniform(vis), uniform(P), uniform(off));
+        });
     }
 
     // epilogue: total over the four lane groups, normalise, base-2 LSE
@@ -679,13 +697,15 @@ template <int DT, int QM, int KVM, int RM, bool MV>
 __global__ __launch_bounds__(256) void dv_stream(const DecodeParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ long long s_scan[4];
-    const int wv = threadIdx.x >> 6;
+    const int wv = uniform((int)(threadIdx.x >> 6));
     const int HPW = p.hpw;
     long long* s_pref = reinterpret_cast<long long*>(smem + HPW * stream::kWaveLds);
     unsigned char* wlds = smem + wv * stream::kWaveLds;
-    run_schedule<true>(p, p.Hkv / HPW, s_pref, s_scan, [&](int row) { return row_visible<KVM, RM>(p, row); },
+    run_schedule<true, KVM == kKvPaged ? kStep : 1>(p, p.Hkv / HPW, s_pref, s_scan, [&](int row) { return row_visible<KVM, RM>(p, row); },
                        [&](int row, int hg, long long v0, long long v1, bool fin, int slot, long long rk) {
-        if (wv < HPW) stream::piece<DT, QM, KVM, RM, MV>(p, wlds, row, hg * HPW + wv, v0, v1, fin, slot, wv, rk);
+        if (wv < HPW)
+            stream::piece<DT, QM, KVM, RM, MV>(p, wlds, uniform(row), uniform(hg) * HPW + wv, uniform(v0), uniform(v1),
+                                               uniform((int)fin) != 0, uniform(slot), wv, uniform(rk));
     });
 }
 
@@ -917,7 +937,7 @@ hipError_t launch_decode(int dtype, int qmode, int kvmode, int rowmode, const De
     unsigned char* ws = reinterpret_cast<unsigned char*>(workspace);
     p.part = reinterpret_cast<float*>(ws);
     p.dir = reinterpret_cast<int*>(ws + part_bytes);
-    p.piece_cost = dtype == kF32 ? 0 : kPieceCost;
+    p.piece_cost = dtype == kF32 ? 0 : kvmode == kKvContig ? kPieceCostContig : kPieceCost;
     // the fp32 kernel waits for each 32-key stage before the next: one stage per
     // workgroup is worth it on small problems
     if (dtype == kF32 && p.min_keys > kStep) p.min_keys = kStep;
@@ -926,7 +946,8 @@ hipError_t launch_decode(int dtype, int qmode, int kvmode, int rowmode, const De
         p.row_begin = r0;
         p.nrows = nrows_total - r0 < kMaxRows ? nrows_total - r0 : kMaxRows;
         // enough workgroups to fill the chip, never more than the key count allows
-        const long long cap = ((long long)p.nrows * nhg * max_keys_per_row + p.min_keys - 1) / p.min_keys;
+        const long long cap =
+            ((long long)p.nrows * nhg * (max_keys_per_row + p.piece_cost) + p.min_keys - 1) / p.min_keys;
         switch (dtype) {
             case kBF16: e = dispatch_modes<kBF16>(qmode, kvmode, rowmode, p, device, max_wg, cap, cus, stream); break;
             case kF16: e = dispatch_modes<kF16>(qmode, kvmode, rowmode, p, device, max_wg, cap, cus, stream); break;

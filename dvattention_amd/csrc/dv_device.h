@@ -81,6 +81,13 @@ __device__ inline void mfma_settle(f32x4 (&o)[8]) {
                  : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]), "+v"(o[4]), "+v"(o[5]), "+v"(o[6]), "+v"(o[7]));
 }
 
+// The same for accumulators kept in AGPRs, where the MFMAs update them in place
+// (operands in VGPRs would be moved out and back in every stage).
+__device__ inline void mfma_settle_acc(f32x4 (&o)[8]) {
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7"
+                 : "+a"(o[0]), "+a"(o[1]), "+a"(o[2]), "+a"(o[3]), "+a"(o[4]), "+a"(o[5]), "+a"(o[6]), "+a"(o[7]));
+}
+
 // ---- memory helpers ---------------------------------------------------------
 
 // 16-byte loads from global memory (address space 1, so the compiler emits
@@ -154,8 +161,24 @@ __device__ inline void wait_vmcnt() {
 // Wait until this wave's LDS operations are complete.
 __device__ inline void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
+// The same with a wave-uniform base address and a 32-bit byte offset per lane.
+__device__ inline void dma16_base(unsigned long long base, uint32_t off, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base),
+                 "s"(lds_base)
+                 : "memory", "m0");
+}
+
 // ---- wave-level helpers -----------------------------------------------------
 
+
+// A wave-uniform value computed per lane, moved to scalar registers.
+__device__ inline int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ inline long long uniform(long long v) {
+    const unsigned long long u = (unsigned long long)v;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+    return (long long)(((unsigned long long)hi << 32) | lo);
+}
 
 // Max / sum over the four 16-lane rows of a wave (lanes n, n+16, n+32, n+48),
 // every lane receiving the result, with the gfx950 row-swap permutes (VALU;

@@ -18,7 +18,8 @@ namespace dv {
 // wave); both give the same chunks.  Workgroup 0 writes
 // the merge directory (segment -> first partial slot, piece count).  Then
 // piece(row, head_group, v0, v1, final, slot, row_keys) runs for each piece of
-// this workgroup's chunk: visible keys [v0, v1) of the segment, `final` when
+// this workgroup's chunk: visible keys [v0, v1) of the segment (cuts inside a
+// segment fall on multiples of kAlign keys), `final` when
 // the segment has no other piece, `slot` its partial slot, `row_keys` the row's
 // visible key count.  Slots are
 // sg + workgroup index, increasing along the cost space, so they are unique and
@@ -34,7 +35,7 @@ __device__ inline long long udiv(long long a, long long b) {
 // per-row cost prefix sums: pref_u(r) for a wave-uniform r, pref_v(r) for a
 // per-lane r (called with every lane active), find_row(u) = the last row r
 // with NHG * pref[r] <= u, total = pref[nrows].
-template <class PrefU, class PrefV, class FindRow, class PieceFn>
+template <int kAlign, class PrefU, class PrefV, class FindRow, class PieceFn>
 __device__ inline void split_chunks(const DecodeParams& p, int NHG, long long total, PrefU&& pref_u, PrefV&& pref_v,
                                     FindRow&& find_row, PieceFn&& piece) {
     const int tid = threadIdx.x;
@@ -50,8 +51,13 @@ __device__ inline void split_chunks(const DecodeParams& p, int NHG, long long to
     //    mille; 0: equal chunks).  Chunk i spans [bound(i), bound(i + 1)).
     const long long Wc = total * NHG;
     const long long ng = udiv(Wc + p.min_keys - 1, p.min_keys);
-    const int geff = Wc == 0 ? 0 : (int)(ng < p.nwg ? ng : p.nwg);
-    const long long chunk = geff ? udiv(Wc + geff - 1, geff) : 1;
+    int geff = Wc == 0 ? 0 : (int)(ng < p.nwg ? ng : p.nwg);
+    long long chunk = geff ? udiv(Wc + geff - 1, geff) : 1;
+    if (kAlign > 1 && chunk < 8 * kAlign) {
+        // short chunks: whole stages, or some of them would take one more
+        chunk = (chunk + kAlign - 1) & ~(long long)(kAlign - 1);
+        geff = (int)udiv(Wc + chunk - 1, chunk);
+    }
     const long long skew = udiv(chunk * p.skew_pm, 1000);
     auto bound = [&](long long i) {
         const long long b = i * chunk + ((i & 1) ? skew : 0);
@@ -111,13 +117,17 @@ __device__ inline void split_chunks(const DecodeParams& p, int NHG, long long to
             // the divisions)
             const bool fin = ka >= u0 && segc + D - 1 < uend;
             const int slot = sg + gidx;  // = first slot of the segment (chunk_of(ka) + sg) + piece index
-            piece(p.row_begin + r, hg, a - ka, b - ka, fin, slot, D - c);
+            // cuts inside a segment move down to a multiple of kAlign keys (both
+            // neighbours use the same rule; a piece may be left without keys)
+            const long long v0 = (a - ka) & ~(long long)(kAlign - 1);
+            const long long v1 = b == segc + D ? b - ka : (b - ka) & ~(long long)(kAlign - 1);
+            piece(p.row_begin + r, hg, v0, v1, fin, slot, D - c);
         }
         u = segc + D;
     }
 }
 
-template <bool kRegPrefix = false, class RowKeys, class PieceFn>
+template <bool kRegPrefix = false, int kAlign = 1, class RowKeys, class PieceFn>
 __device__ inline void run_schedule(const DecodeParams& p, int NHG, long long* s_pref, long long* s_scan,
                                     RowKeys&& row_keys, PieceFn&& piece) {
     const int tid = threadIdx.x;
@@ -143,13 +153,18 @@ __device__ inline void run_schedule(const DecodeParams& p, int NHG, long long* s
             d = v > 0 ? v + c : 0;
         }
         long long incl = d;
-#pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) {
+        // steps past the row count add nothing (a single row takes none)
+#pragma unroll 1
+        for (int o = 1; o < nrows; o <<= 1) {
             const long long t = __shfl_up(incl, o, kWave);
             if (lane >= o) incl += t;
         }
-        excl = incl - d;
-        total = __shfl(incl, kWave - 1, kWave);
+        const int last = nrows - 1;
+        total = (long long)(((unsigned long long)(uint32_t)__builtin_amdgcn_readlane(
+                                 (int)(uint32_t)((unsigned long long)incl >> 32), last)
+                             << 32) |
+                            (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)incl, last));
+        excl = lane < nrows ? incl - d : total;
     } else {
         const int per = (nrows + nthreads - 1) / nthreads;
         const int r0 = tid * per;
@@ -210,7 +225,7 @@ __device__ inline void run_schedule(const DecodeParams& p, int NHG, long long* s
         }
         return lo;
     };
-    split_chunks(p, NHG, total, pref_u, pref_v, find_row, piece);
+    split_chunks<kAlign>(p, NHG, total, pref_u, pref_v, find_row, piece);
 }
 
 }  // namespace dv

@@ -438,10 +438,12 @@ inline int pick_hpw(int Hkv) {
 }
 
 // Start cost of a piece in the 16-bit decode's work split, in keys: about the
-// time a workgroup needs to restart its pipeline on a new segment (measured
-// against 64, 96, 128 and 160: configurations 2 and 3 ran fastest at 192,
-// configuration 4 within its spread).
-constexpr int kPieceCost = 192;
+// time a workgroup needs to restart its pipeline on a new segment.  Paged calls,
+// one view / 2-4 views / one sequence of 3001 keys: 98.0 / 89.5 / 17.1 us with
+// 128, 97.9 / 87.7 / 16.9 with 160, 98.4 / 88.5 / 17.0 with 192.  Contiguous
+// calls of several short views: 30.4 us with 192, 31.6 with 160.
+constexpr int kPieceCost = 160;
+constexpr int kPieceCostContig = 192;
 
 // Smallest key range worth a workgroup in the decode split.
 constexpr int kDecodeMinKeys = 64;
@@ -474,8 +476,15 @@ __device__ inline void fill_pages(const DecodeParams& p, const int* bt, int* pc,
     constexpr int kIt = kPc / kWave;
     const int lane = threadIdx.x & 63;
     const uint32_t maxB = (uint32_t)p.maxB;
-    const int nk = (n + kWave - 1) / kWave;  // passes with entries (wave-uniform)
     if (n <= 0) return;
+    if (n <= kWave) {  // one pass: most pieces of a small call
+        const uint32_t lp = lp_of(lane < n ? lane : n - 1);
+        int v = maxB > 0 ? bt[lp < maxB ? lp : maxB - 1] : -1;
+        if (lp >= maxB || v < 0 || v >= p.nblocks) v = -1;
+        if (lane < n) pc[lane] = v;
+        return;
+    }
+    const int nk = (n + kWave - 1) / kWave;  // passes with entries (wave-uniform)
     int pg[kIt];
     uint32_t ok = 0;  // bit k: entry lane + 64k exists and lies in the row
 #pragma unroll
@@ -502,7 +511,7 @@ struct View {
     const unsigned char* v;
     int off;                 // paged: logical position of the view's key 0
     int lp0;                 // paged: logical page of page-cache entry 0
-    int b;                   // end (exclusive) of the current view-local key range
+    int a, b;                // current view-local key range [a, b)
     int hkv;
 };
 
@@ -527,13 +536,13 @@ __device__ inline uint32_t issue(const DecodeParams& p, const View& v, const int
             uint32_t lp, r;
             page_split(p, pos > 0 ? (uint32_t)pos : 0u, lp, r);
             const uint32_t idx = lp - (uint32_t)v.lp0;
-            const bool in = key < v.b && pos >= 0 && idx < (uint32_t)kPc;
+            const bool in = key >= v.a && key < v.b && pos >= 0 && idx < (uint32_t)kPc;
             const int page = in ? pc[in ? idx : 0u] : -1;
             ok[i] = page >= 0;
             const uint32_t rowidx = ((uint32_t)page * (uint32_t)p.bs + r) * (uint32_t)p.Hkv + (uint32_t)v.hkv;
             boff = (unsigned long long)rowidx << 8;
         } else {
-            ok[i] = key < v.b;
+            ok[i] = key >= v.a && key < v.b;
             boff = (unsigned long long)(uint32_t)key << 8;
         }
         const int gk = c16 ^ (kk & 15), gv = c16 ^ ((kk & 7) << 1);
@@ -551,6 +560,74 @@ __device__ inline uint32_t issue(const DecodeParams& p, const View& v, const int
         mask |= bits << (i * 4);
     }
     return mask;
+}
+
+// First key of the stages of a view whose range starts at key l0: paged stages
+// start at a multiple of 32 logical positions (possibly before the view; such
+// keys are invisible), so that with pages of a multiple of 16 keys each half of
+// a stage lies in one page.
+template <int KVM>
+__device__ inline int stage_start(int off, int l0) {
+    return KVM == kKvPaged ? l0 - ((off + l0) & (kStep - 1)) : l0;
+}
+
+// This lane's byte offsets from the row base of a full stage's loads: load i
+// moves key rows 4i .. 4i + 3 (lane / 16), whose swizzles repeat every four (K)
+// and two (V) loads.
+struct LaneOff {
+    uint32_t k[4], v[2];
+};
+
+__device__ inline LaneOff lane_offsets(uint32_t row_stride) {
+    const int lane = threadIdx.x & 63;
+    const int c16 = lane & 15, sub = lane >> 4;
+    LaneOff o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o.k[i] = (uint32_t)sub * row_stride + (uint32_t)((c16 ^ (i * 4 + sub)) * 16);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) o.v[i] = (uint32_t)sub * row_stride + (uint32_t)((c16 ^ ((i * 4 + sub) << 1)) * 16);
+    return o;
+}
+
+// issue() of a paged stage that may be full: a stage whose 32 keys are all
+// visible, in pages of a power of two of at least 16 keys, needs no lane to look
+// up its rows: the two pages are read once for the wave, the row bases are scalar
+// and every load is a scalar base plus a lane constant -- about 120 instructions,
+// none of them vector arithmetic, where issue() takes 130 vector and 120 scalar
+// ones (one wave per SIMD: each is time the stage's loads and MFMAs wait for).
+// Everything but the lane offsets is wave-uniform.
+__device__ inline uint32_t issue_stage(const DecodeParams& p, const View& v, const LaneOff& lo, const int* pc,
+                                       uint32_t sbase, int l) {
+    if (l >= v.a && l + kStep <= v.b && p.bs_shift >= 4) {
+        const uint32_t pos = (uint32_t)(v.off + l), in = (1u << p.bs_shift) - 1u;
+        const int pg0 = uniform(pc[(int)(pos >> p.bs_shift) - v.lp0]);
+        const int pg1 = uniform(pc[(int)((pos + 16) >> p.bs_shift) - v.lp0]);
+        if (pg0 >= 0 && pg1 >= 0) {
+            const uint32_t r0 = ((uint32_t)pg0 << p.bs_shift) + (pos & in);  // cache rows of keys l and l + 16
+            const uint32_t r1 = ((uint32_t)pg1 << p.bs_shift) + ((pos + 16) & in);
+            const unsigned long long row[2] = {(unsigned long long)(r0 * (uint32_t)p.Hkv + (uint32_t)v.hkv) << 8,
+                                               (unsigned long long)(r1 * (uint32_t)p.Hkv + (uint32_t)v.hkv) << 8};
+            const unsigned long long kb = (unsigned long long)v.k, vb = (unsigned long long)v.v;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const unsigned long long r = row[i >> 2] + (unsigned long long)((uint32_t)(i & 3) * ((uint32_t)p.Hkv << 10));
+                dma16_base(kb + r, lo.k[i & 3], sbase + (uint32_t)(i * 1024));
+                dma16_base(vb + r, lo.v[i & 1], sbase + (uint32_t)(kTile + i * 1024));
+            }
+            return 0xffffffffu;
+        }
+    }
+    return (uint32_t)uniform((int)issue<kKvPaged>(p, v, pc, sbase, l));
+}
+
+// A stage of either kind.  Contiguous views keep the one general path: their
+// pieces end anywhere in a stage, and a short call pays for every path whose
+// code it fetches (four rows over 4.5k keys: 17.1 us with both, 15.6 with one).
+template <int KVM>
+__device__ inline uint32_t issue_keys(const DecodeParams& p, const View& v, const LaneOff& lo, const int* pc,
+                                      uint32_t sbase, int l) {
+    if constexpr (KVM == kKvPaged) return issue_stage(p, v, lo, pc, sbase, l);
+    else return issue<KVM>(p, v, pc, sbase, l);
 }
 
 }  // namespace stream

@@ -1,0 +1,42 @@
+"""Paged decode of one token against the oracle at the lengths and page sizes
+where a stage of 32 keys takes one load path or the other
+(dvattention_amd/csrc/dv_stream.h, issue_stage): pages of 8, 16, 24, 32 and 64
+keys, ranges that start and end inside a stage, views that start off a multiple
+of 32 logical positions, and rows short enough that a cut leaves a piece without
+keys.  Tolerances: test_gpu_parity.close."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import dvattn_oracle as O
+from test_gpu_parity import close, dv, rand_paged, run_paged  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bs", [8, 16, 24, 32, 64])
+@pytest.mark.parametrize("W,Hkv,lens", [(1, 1, [1]), (1, 4, [31]), (2, 2, [32]), (1, 8, [3001]), (3, 4, [65]),
+                                        (2, 4, [37, 100, 5]), (66, 4, [130]), (2, 1, [9000])])
+def test_paged_stage_paths(dv, gpu, dtype, bs, W, Hkv, lens):  # noqa: F811
+    F = len(lens)
+    rng = np.random.default_rng(bs + sum(lens))
+    loc = np.array(lens)[:, None, None] - 1 - rng.integers(0, min(lens), size=(F, W, 1))
+    d = rand_paged(F, W, 1, Hkv, bs, lens, 64, dtype, seed=bs, loc=loc, k_scale=1.5)
+    close(run_paged(dv, d, 0.1, gpu), O.paged_sdpa(0.1, **d), dtype, f"bs={bs} {lens}")
+
+
+@pytest.mark.parametrize("bs", [16, 32])
+def test_invalid_page_in_a_full_stage(dv, gpu, bs):  # noqa: F811
+    # a page outside the pool in the middle of a row: its keys are masked, the
+    # stage's other keys are not
+    d = rand_paged(1, 1, 1, 1, bs, [320], 64, torch.bfloat16, seed=3, loc=np.array([[[319]]]))
+    bt = d["block_tables"].clone()
+    bt[0, 3] = 10 ** 6
+    out = run_paged(dv, dict(d, block_tables=bt), 0.1, gpu).cpu()
+    pos = np.array([i for i in range(320) if i // bs != 3])
+    pages = d["block_tables"][0].numpy()[pos // bs]
+    rq = O.rope_q(d["queries"], d["cosines"], d["sines"])[0, 0, :, 0].float()
+    k = d["k_cache"][pages, pos % bs, 0].float()
+    v = d["v_cache"][pages, pos % bs, 0].float()
+    close(out[0, :, 0], torch.softmax(0.1 * (rq @ k.T), -1) @ v, torch.bfloat16, f"bs={bs}")
