@@ -9,7 +9,8 @@
 //  * Workgroup = eight waves, two per SIMD, on one (sequence, 16-token block,
 //    KV head) and a contiguous range of its visible keys.  Wave w owns tokens
 //    2w and 2w+1: two 16-row query tiles (16 heads each), so a K/V stage read
-//    from LDS feeds 32 query rows per wave and 256 per workgroup.
+//    from LDS feeds 32 query rows per wave and 256 per workgroup.  Groups of at
+//    most eight tokens split the keys instead (KS wave sets, stream_range).
 //  * K/V pages stream through an 8-stage LDS ring filled by direct-to-LDS loads
 //    (global_load_lds_dwordx4, non-temporal): 32 keys x 256 B of K and of V per
 //    stage, one eighth issued by each wave, seven stages ahead of the one

@@ -945,7 +945,8 @@ hipError_t launch_decode(int dtype, int qmode, int kvmode, int rowmode, const De
     for (int r0 = 0; r0 < nrows_total; r0 += kMaxRows) {
         p.row_begin = r0;
         p.nrows = nrows_total - r0 < kMaxRows ? nrows_total - r0 : kMaxRows;
-        // enough workgroups to fill the chip, never more than the key count allows
+        // enough workgroups to fill the chip, never more than the keys and the start
+        // costs allow (without the latter a small call's chunks end past a stage)
         const long long cap =
             ((long long)p.nrows * nhg * (max_keys_per_row + p.piece_cost) + p.min_keys - 1) / p.min_keys;
         switch (dtype) {

@@ -54,7 +54,8 @@ __device__ inline void split_chunks(const DecodeParams& p, int NHG, long long to
     int geff = Wc == 0 ? 0 : (int)(ng < p.nwg ? ng : p.nwg);
     long long chunk = geff ? udiv(Wc + geff - 1, geff) : 1;
     if (kAlign > 1 && chunk < 8 * kAlign) {
-        // short chunks: whole stages, or some of them would take one more
+        // short chunks: whole stages, or some of them would take one more (one
+        // sequence of 3001 keys in chunks of 68 keys: 18.1 us, of 64: 16.9)
         chunk = (chunk + kAlign - 1) & ~(long long)(kAlign - 1);
         geff = (int)udiv(Wc + chunk - 1, chunk);
     }
