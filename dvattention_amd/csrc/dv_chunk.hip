@@ -997,7 +997,12 @@ hipError_t launch_varlen_chunk(int dtype, const DecodeParams& base, long long ma
     // (2 x 64 tokens, 500 keys, 8 KV heads: 43.5 -> 48.3 us; 4 x 4 x 500: 31.4 ->
     // 36.8), the split saves a quarter of a call of short ones (32 x 4 x 4608
     // keys: 185 -> 124 us)
-    const int ks = dtype == kF32 || base.W * (long long)base.Hkv * max_keys_per_group < kFewMinKeys
+    // T a multiple of W: taken for a uniform batch, which has short groups only if
+    // its token count per sequence ends in one (16 x 16 tokens, 8208 keys: 179 us
+    // with one launch, 184-190 with an empty second one)
+    const int rem = base.T / base.W % chunk::kTokBlk;
+    const bool no_short = base.T % base.W == 0 && (rem == 0 || rem > chunk::kFewTok);
+    const int ks = dtype == kF32 || no_short || base.W * (long long)base.Hkv * max_keys_per_group < kFewMinKeys
                        ? 1
                        : chunk::key_split(base.l2scale, chunk::kFewTok);
     const int few = ks > 1 ? chunk::kFewTok : 0;
