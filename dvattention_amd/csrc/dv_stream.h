@@ -571,6 +571,14 @@ __device__ inline int stage_start(int off, int l0) {
     return KVM == kKvPaged ? l0 - ((off + l0) & (kStep - 1)) : l0;
 }
 
+// Whether the two pages (of 2^shift keys) of the stage at logical position pos,
+// a multiple of 16, have entries in the page cache, whose entry 0 is page lp0.
+__host__ __device__ inline bool full_stage_in_cache(int pos, int shift, int lp0) {
+    const uint32_t i0 = ((uint32_t)pos >> shift) - (uint32_t)lp0;
+    const uint32_t i1 = (((uint32_t)pos + 16u) >> shift) - (uint32_t)lp0;
+    return pos >= 0 && i0 < (uint32_t)kPc && i1 < (uint32_t)kPc;
+}
+
 // This lane's byte offsets from the row base of a full stage's loads: load i
 // moves key rows 4i .. 4i + 3 (lane / 16), whose swizzles repeat every four (K)
 // and two (V) loads.
@@ -596,10 +604,14 @@ __device__ inline LaneOff lane_offsets(uint32_t row_stride) {
 // none of them vector arithmetic, where issue() takes 130 vector and 120 scalar
 // ones (one wave per SIMD: each is time the stage's loads and MFMAs wait for).
 // Everything but the lane offsets is wave-uniform.
+// A stage that reaches outside the page cache goes to issue(), which masks such
+// keys: positions below 0 (a negative fragment length before the view; lengths
+// are device data) have no entry.
 __device__ inline uint32_t issue_stage(const DecodeParams& p, const View& v, const LaneOff& lo, const int* pc,
                                        uint32_t sbase, int l) {
-    if (l >= v.a && l + kStep <= v.b && p.bs_shift >= 4) {
-        const uint32_t pos = (uint32_t)(v.off + l), in = (1u << p.bs_shift) - 1u;
+    const int pos0 = v.off + l;
+    if (l >= v.a && l + kStep <= v.b && p.bs_shift >= 4 && full_stage_in_cache(pos0, p.bs_shift, v.lp0)) {
+        const uint32_t pos = (uint32_t)pos0, in = (1u << p.bs_shift) - 1u;
         const int pg0 = uniform(pc[(int)(pos >> p.bs_shift) - v.lp0]);
         const int pg1 = uniform(pc[(int)((pos + 16) >> p.bs_shift) - v.lp0]);
         if (pg0 >= 0 && pg1 >= 0) {
