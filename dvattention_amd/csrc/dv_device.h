@@ -152,6 +152,19 @@ __device__ inline void dma16(const void* gptr, uint32_t lds_base) {
                  : "memory", "m0");
 }
 
+// dma16 of a K and a V piece, each with a wave-uniform base address and a 32-bit
+// byte offset per lane.  A vector-memory instruction may read a scalar register
+// only five wait states after a vector instruction (v_readfirstlane, v_readlane)
+// wrote it, and the compiler does not look for that inside the asm, so the wait
+// is part of it, whatever produced the bases; it covers both loads.
+__device__ inline void dma16_kv(unsigned long long kbase, uint32_t koff, uint32_t klds, unsigned long long vbase,
+                                uint32_t voff, uint32_t vlds) {
+    asm volatile("s_mov_b32 m0, %4\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1 nt\n\t"
+                 "s_mov_b32 m0, %5\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3 nt" ::"v"(koff),
+                 "s"(kbase), "v"(voff), "s"(vbase), "s"(klds), "s"(vlds)
+                 : "memory", "m0");
+}
+
 // Wait until at most N vector-memory operations of this wave are outstanding.
 template <int N>
 __device__ inline void wait_vmcnt() {
@@ -160,13 +173,6 @@ __device__ inline void wait_vmcnt() {
 
 // Wait until this wave's LDS operations are complete.
 __device__ inline void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
-// The same with a wave-uniform base address and a 32-bit byte offset per lane.
-__device__ inline void dma16_base(unsigned long long base, uint32_t off, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base),
-                 "s"(lds_base)
-                 : "memory", "m0");
-}
 
 // ---- wave-level helpers -----------------------------------------------------
 

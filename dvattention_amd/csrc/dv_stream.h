@@ -623,8 +623,8 @@ __device__ inline uint32_t issue_stage(const DecodeParams& p, const View& v, con
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const unsigned long long r = row[i >> 2] + (unsigned long long)((uint32_t)(i & 3) * ((uint32_t)p.Hkv << 10));
-                dma16_base(kb + r, lo.k[i & 3], sbase + (uint32_t)(i * 1024));
-                dma16_base(vb + r, lo.v[i & 1], sbase + (uint32_t)(kTile + i * 1024));
+                dma16_kv(kb + r, lo.k[i & 3], sbase + (uint32_t)(i * 1024), vb + r, lo.v[i & 1],
+                         sbase + (uint32_t)(kTile + i * 1024));
             }
             return 0xffffffffu;
         }
