@@ -171,6 +171,16 @@ __device__ inline long long group_visible(const DecodeParams& p, int rg) {
     return total;
 }
 
+// Logical page of a position, as the page cache counts them: an end of a key
+// range below 0 (a negative fragment length before the view; lengths are device
+// data) or past 32 bits counts as the nearest position there is, so the first
+// page of a range is never after its last; row_of finds no entry for such keys.
+__device__ inline bool position_in_range(long long pos) { return pos >= 0 && pos <= (long long)UINT32_MAX; }
+__device__ inline uint32_t logical_page(const DecodeParams& p, long long pos) {
+    const uint32_t u = pos < 0 ? 0u : pos > (long long)UINT32_MAX ? UINT32_MAX : (uint32_t)pos;
+    return p.bs_shift >= 0 ? u >> p.bs_shift : u / (uint32_t)p.bs;
+}
+
 // Page-cache fill of a chunk workgroup (kThreads threads), in two parts so that
 // other loads can be issued between: pages[i] = entry lp0 + i of the sequence's
 // block_tables row bt, for the entries up to logical page lpl (-1 past the row or

@@ -614,9 +614,8 @@ __device__ void chunk_piece(const DecodeParams& p, unsigned char* smem, int* pag
                 uint32_t lpl = 0;
                 r.lp0 = 0;
                 if (KVM == kKvPaged) {
-                    const uint32_t p0 = (uint32_t)(off + sa), p1 = (uint32_t)(off + sbnd - 1);
-                    lpl = p.bs_shift >= 0 ? (p1 >> p.bs_shift) : p1 / (uint32_t)p.bs;
-                    r.lp0 = p.bs_shift >= 0 ? (p0 >> p.bs_shift) : p0 / (uint32_t)p.bs;
+                    lpl = logical_page(p, off + sbnd - 1);
+                    r.lp0 = logical_page(p, off + sa);
                     fetch_pages(p, p.bt + (long long)w * p.maxB, r.lp0, lpl, pg);
                 }
                 // the ring is idle here (previous range drained): stage the query tiles
@@ -628,10 +627,12 @@ __device__ void chunk_piece(const DecodeParams& p, unsigned char* smem, int* pag
                         ntile, kg, f, hkv);
                     if (KS == 1) read_q_tiles(qreg, ntile, qB);
                 }
-                // every page of the sub-range is valid; the page ids are written and the
-                // query tiles read (KS > 1: staged)
+                // every position and page of the sub-range is valid; the page ids are
+                // written and the query tiles read (KS > 1: staged)
                 bool ok = true;
-                if (KVM == kKvPaged) ok = store_pages(p, pages, r.lp0, lpl, pg);
+                if (KVM == kKvPaged)
+                    ok = store_pages(p, pages, r.lp0, lpl, pg) && position_in_range(off + sa) &&
+                         position_in_range(off + sbnd - 1);
                 r.pages_ok = __syncthreads_and(ok) != 0;
                 if (KS > 1 && sa == la) {
                     read_q_tiles(qreg, ntile, qB);

@@ -15,9 +15,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("bs", [16, 24, 64])
+@pytest.mark.parametrize("S", [1, 4, 17])
 @pytest.mark.parametrize("neg,n", [(32, 200), (64, 96), (100, 3000), (70, 64), (4096, 5000)])
-def test_view_at_a_negative_position(dv, gpu, dtype, bs, neg, n):  # noqa: F811
-    W, Hkv, S = 2, 2, 1
+def test_view_at_a_negative_position(dv, gpu, dtype, bs, neg, n, S):  # noqa: F811
+    W, Hkv = 2, 2
     loc = np.stack([np.full((W, S), -1), n - S + np.arange(S)[None].repeat(W, 0)])
     d = rand_paged(2, W, S, Hkv, bs, [0, n], 64, dtype, seed=neg + bs, loc=loc)
     out = run_paged(dv, dict(d, fragment_lengths=torch.tensor([-neg, n], dtype=torch.int32)), 0.1, gpu)
@@ -25,4 +26,4 @@ def test_view_at_a_negative_position(dv, gpu, dtype, bs, neg, n):  # noqa: F811
     seen = max(0, n - neg)
     want = O.paged_sdpa(0.1, **dict(d, locations=torch.from_numpy(np.maximum(loc - neg, -1).astype(np.int32)),
                                     fragment_lengths=torch.tensor([0, seen], dtype=torch.int32)))
-    close(out, want, dtype, f"bs={bs} -{neg} {n}")
+    close(out, want, dtype, f"bs={bs} -{neg} {n} S={S}")
