@@ -525,14 +525,16 @@ __device__ inline void combine_split(unsigned char* smem, int wv, int kg, int nt
                 mk[k] = reinterpret_cast<const float*>(rec(k, t) + 8 * 1024)[lane];
                 M = fmaxf(M, mk[k]);
             }
-            if (M == -DV_INF) continue;  // no visible key in any subset
-            const float s0 = __builtin_amdgcn_exp2f(tl[t].m - M);  // an empty subset (-inf) -> 0
+            // an empty subset (-inf) -> weight 0; with no maximum in any, all have
+            // it, and what a NaN left in a subset's sums stays
+            const float Mf = M == -DV_INF ? 0.0f : M;
+            const float s0 = __builtin_amdgcn_exp2f(tl[t].m - Mf);
             tl[t].l *= s0;
 #pragma unroll
             for (int c = 0; c < 8; ++c) tl[t].o[c] *= s0;
 #pragma unroll
             for (int k = 1; k < KS; ++k) {
-                const float sk = __builtin_amdgcn_exp2f(mk[k] - M);
+                const float sk = __builtin_amdgcn_exp2f(mk[k] - Mf);
                 tl[t].l += sk * reinterpret_cast<const float*>(rec(k, t) + 8 * 1024)[64 + lane];
 #pragma unroll
                 for (int c = 0; c < 8; ++c)

@@ -55,3 +55,15 @@ def test_varlen_mixed_unsorted_table(dv, gpu):  # noqa: F811
     # a table that is not non-decreasing, and tokens past its last entry
     d = rand_varlen(2, 4, 45, np.array([0, 3, 2, 30, 29]), 1, 16, [60, 200], 32, torch.bfloat16, seed=5)
     close(run_varlen(dv, d, 0.1, gpu), O.varlen_paged_sdpa(0.1, **d), torch.bfloat16, "unsorted")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("S", [2, 4, 8, 9])
+def test_nan_beside_an_empty_wave_set(dv, gpu, dtype, S):  # noqa: F811
+    # the first wave set's keys have no page, another set's keys are NaN: one piece
+    # gives NaN with and without the split (S = 9)
+    d = rand_paged(1, 1, S, 1, 32, [64], 64, dtype, seed=S, loc=np.full((1, 1, S), 63))
+    bt, kc = d["block_tables"].clone(), d["k_cache"].clone()
+    kc[bt[0, 1]] = float("nan")
+    bt[0, 0] = 10 ** 6
+    assert run_paged(dv, dict(d, block_tables=bt, k_cache=kc), 0.1, gpu).isnan().all()
