@@ -379,7 +379,7 @@ __device__ bool views_stream(const DecodeParams& p, unsigned char* wlds, int row
                              long long v1, uint64_t vm, const ViewTab& t, SoftState& st) {
     const uint32_t ring = __builtin_amdgcn_readfirstlane(lds_addr(wlds));
     int* pc = reinterpret_cast<int*>(wlds + kRing * kStage);
-    int vf[kStreamViews], ls[kStreamViews], l0[kStreamViews], l1[kStreamViews], ns[kStreamViews], pcb[kStreamViews + 1];
+    int vf[kStreamViews], l0[kStreamViews], l1[kStreamViews], ns[kStreamViews], pcb[kStreamViews + 1];
     int voff[kStreamViews], lpa[kStreamViews];
     int npages = 0, N = 0;
     uint64_t m = vm;
@@ -397,14 +397,13 @@ __device__ bool views_stream(const DecodeParams& p, unsigned char* wlds, int row
         l0[j] = has ? (int)(a - P) : 0;
         l1[j] = has ? (int)(b - P) : 0;
         voff[j] = (int)off;
-        ls[j] = has ? stage_start<kKvPaged>(voff[j], l0[j]) : 0;
-        ns[j] = (l1[j] - ls[j] + kStep - 1) / kStep;
+        ns[j] = (l1[j] - l0[j] + kStep - 1) / kStep;
         N += ns[j];
         lpa[j] = 0;
         pcb[j] = npages;
         if (has) {
             uint32_t la, lz, r;
-            const int pa = voff[j] + ls[j], pz = voff[j] + l1[j] - 1;
+            const int pa = voff[j] + l0[j], pz = voff[j] + l1[j] - 1;
             page_split(p, pa > 0 ? (uint32_t)pa : 0u, la, r);
             page_split(p, pz > 0 ? (uint32_t)pz : 0u, lz, r);
             lpa[j] = (int)la;
@@ -445,11 +444,9 @@ __device__ bool views_stream(const DecodeParams& p, unsigned char* wlds, int row
     vi.v = reinterpret_cast<const unsigned char*>(p.vc);
     vi.off = voff[0];
     vi.lp0 = lpa[0];
-    vi.a = l0[0];
     vi.b = l1[0];
-    const LaneOff lo = lane_offsets((uint32_t)p.Hkv << 8);
     const int* pci = pc;
-    int ji = 0, li = ls[0];
+    int ji = 0, li = l0[0];
     auto advance = [&]() {
         li += kStep;
         if (li >= vi.b) {
@@ -459,18 +456,17 @@ __device__ bool views_stream(const DecodeParams& p, unsigned char* wlds, int row
                 if (k == ji) {
                     vi.off = voff[k];
                     vi.lp0 = lpa[k];
-                    vi.a = l0[k];
                     vi.b = l1[k];
                     pci = pc + pcb[k];
-                    li = ls[k];
+                    li = l0[k];
                 }
         }
     };
-    uint32_t m0 = issue_stage(p, vi, lo, pci, ring, li);
+    uint32_t m0 = issue<kKvPaged>(p, vi, pci, ring, li);
     advance();
     uint32_t m1 = 0;
     if (N > 1) {
-        m1 = issue_stage(p, vi, lo, pci, ring + kStage, li);
+        m1 = issue<kKvPaged>(p, vi, pci, ring + kStage, li);
         advance();
     }
     // rotated queries of every view while the first stages are in flight, then
@@ -502,7 +498,7 @@ __device__ bool views_stream(const DecodeParams& p, unsigned char* wlds, int row
         compute<DT>(st, kt, kt + kTile, (s & 1) ? m1 : m0, qc, p.l2scale);
         if (s + 2 < N) {
             lds_wait();  // the slot's reads are complete before it is refilled
-            const uint32_t mk = issue_stage(p, vi, lo, pci, ring + (uint32_t)((s & 1) * kStage), li);
+            const uint32_t mk = issue<kKvPaged>(p, vi, pci, ring + (uint32_t)((s & 1) * kStage), li);
             advance();
             if (s & 1) m1 = mk;
             else m0 = mk;
@@ -525,8 +521,8 @@ __device__ bool views_stream(const DecodeParams& p, unsigned char* wlds, int row
 // One wave: KV head hkv over visible keys [v0, v1) of one row.  wlds: this
 // wave's LDS (ring, then page cache).  MV: paged rows of several views stream
 // them back to back (a separate instantiation, so single-view launches keep
-// their own register allocation).
-template <int DT, int QM, int KVM, int RM, bool MV>
+// their own register allocation).  P2: one paged view, see issue_stage.
+template <int DT, int QM, int KVM, int RM, bool MV, bool P2>
 __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int hkv, long long v0, long long v1,
                       bool final_out, int slot, int wv, long long row_keys) {
     const int lane = threadIdx.x & 63;
@@ -570,7 +566,6 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
             const int l0 = (int)(a - P), l1 = (int)(bnd - P);
             View v;
             v.hkv = hkv;
-            v.a = l0;
             const LaneOff lo = lane_offsets(KVM == kKvPaged ? (uint32_t)p.Hkv << 8 : 256u);
             if (KVM == kKvPaged) {
                 v.k = reinterpret_cast<const unsigned char*>(p.kc);
@@ -596,7 +591,7 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
                 span = ((long long)(kPc - 2) * p.bs) & ~(long long)(kStep - 1);
                 span = span < (1ll << 30) ? span : 1ll << 30;
             }
-            for (int sa = stage_start<KVM>(v.off, l0); sa < l1;) {
+            for (int sa = l0; sa < l1;) {
                 const int sb = (long long)l1 - sa > span ? (int)(sa + span) : l1;
                 v.b = sb;
                 if (KVM == kKvPaged) {
@@ -612,13 +607,23 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
                 const int n_st = (sb - sa + kStep - 1) / kStep;
                 // the first two stages in a rolled loop: this code runs once per piece,
                 // and a second copy of it would be fetched cold
+                // the first two stages; a contiguous call's in a rolled loop (its code runs
+                // once per piece, and a second copy of it would be fetched cold: 16 rows
+                // of 2000 keys 33.0 us, 33.4 with two copies), which costs paged calls
+                // more in the stage loop below (32 ragged sequences, pages of 24 keys:
+                // 110.4 us, 100.4 with two copies; 16 keys: 98.7 / 97.7)
                 uint32_t m0 = 0, m1 = 0;
+                if constexpr (KVM == kKvContig) {
 #pragma unroll 1
-                for (int s = 0; s < 2 && s < n_st; ++s) {
-                    m0 = m1;
-                    m1 = issue_keys<KVM>(p, v, lo, pc, ring + (uint32_t)(s * kStage), sa + s * kStep);
+                    for (int s = 0; s < 2 && s < n_st; ++s) {
+                        m0 = m1;
+                        m1 = issue_keys<KVM, P2>(p, v, lo, pc, ring + (uint32_t)(s * kStage), sa + s * kStep);
+                    }
+                    if (n_st == 1) m0 = m1;
+                } else {
+                    m0 = issue_keys<KVM, P2>(p, v, lo, pc, ring, sa);
+                    if (n_st > 1) m1 = issue_keys<KVM, P2>(p, v, lo, pc, ring + kStage, sa + kStep);
                 }
-                if (n_st == 1) m0 = m1;
                 if (!have_q) {
                     // rotated once per (row, view) while the first stages are in flight
                     if (qsplit) rotate_q16<DT, QM>(qr, qB);
@@ -636,7 +641,7 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
                     compute<DT>(st, kt, kt + kTile, (s & 1) ? m1 : m0, qB, p.l2scale);
                     if (s + 2 < n_st) {
                         lds_wait();  // the slot's reads are complete before it is refilled
-                        const uint32_t mk = issue_keys<KVM>(p, v, lo, pc, ring + (uint32_t)((s & 1) * kStage),
+                        const uint32_t mk = issue_keys<KVM, P2>(p, v, lo, pc, ring + (uint32_t)((s & 1) * kStage),
                                                        sa + (s + 2) * kStep);
                         if (s & 1) m1 = mk;
                         else m0 = mk;
@@ -693,7 +698,7 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
 
 }  // namespace stream
 
-template <int DT, int QM, int KVM, int RM, bool MV>
+template <int DT, int QM, int KVM, int RM, bool MV, bool P2>
 __global__ __launch_bounds__(256) void dv_stream(const DecodeParams p) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ long long s_scan[4];
@@ -701,10 +706,10 @@ __global__ __launch_bounds__(256) void dv_stream(const DecodeParams p) {
     const int HPW = p.hpw;
     long long* s_pref = reinterpret_cast<long long*>(smem + HPW * stream::kWaveLds);
     unsigned char* wlds = smem + wv * stream::kWaveLds;
-    run_schedule<true, KVM == kKvPaged ? kStep : 1>(p, p.Hkv / HPW, s_pref, s_scan, [&](int row) { return row_visible<KVM, RM>(p, row); },
+    run_schedule<true, P2 ? kStep : 1>(p, p.Hkv / HPW, s_pref, s_scan, [&](int row) { return row_visible<KVM, RM>(p, row); },
                        [&](int row, int hg, long long v0, long long v1, bool fin, int slot, long long rk) {
         if (wv < HPW)
-            stream::piece<DT, QM, KVM, RM, MV>(p, wlds, uniform(row), uniform(hg) * HPW + wv, uniform(v0), uniform(v1),
+            stream::piece<DT, QM, KVM, RM, MV, P2>(p, wlds, uniform(row), uniform(hg) * HPW + wv, uniform(v0), uniform(v1),
                                                uniform((int)fin) != 0, uniform(slot), wv, uniform(rk));
     });
 }
@@ -815,10 +820,10 @@ int wgs_per_cu(int hpw) { return 8 / hpw; }
 
 // The decode kernel for a dtype: the LDS-streaming kernel for 16-bit types,
 // the register-staged one for fp32.
-template <int DT, int QM, int KVM, int RM, bool MV>
+template <int DT, int QM, int KVM, int RM, bool MV, bool P2>
 const void* decode_kernel() {
     if constexpr (DT == kF32) return reinterpret_cast<const void*>(&dv_decode<DT, QM, KVM, RM>);
-    else return reinterpret_cast<const void*>(&dv_stream<DT, QM, KVM, RM, MV>);
+    else return reinterpret_cast<const void*>(&dv_stream<DT, QM, KVM, RM, MV, P2>);
 }
 
 template <int DT>
@@ -828,7 +833,7 @@ size_t wave_lds() {
 
 // Resident workgroups per CU for one kernel instance at a given dynamic LDS
 // size, cached per 1 KiB of LDS (hipOccupancy queries cost host time).
-template <int DT, int QM, int KVM, int RM, bool MV>
+template <int DT, int QM, int KVM, int RM, bool MV, bool P2>
 int resident_wgs(int hpw, size_t lds) {
     static std::atomic<int> cache[4][161];  // [hpw-1][lds KiB]; 0 = not queried yet
     const int kib = (int)((lds + 1023) / 1024);
@@ -836,7 +841,7 @@ int resident_wgs(int hpw, size_t lds) {
     std::atomic<int>& slot = cache[hpw - 1][kib];
     int nb = slot.load(std::memory_order_relaxed);
     if (nb == 0) {
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, decode_kernel<DT, QM, KVM, RM, MV>(), hpw * kWave,
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, decode_kernel<DT, QM, KVM, RM, MV, P2>(), hpw * kWave,
                                                          (size_t)kib * 1024) != hipSuccess ||
             nb < 1)
             nb = 1;
@@ -845,10 +850,10 @@ int resident_wgs(int hpw, size_t lds) {
     return nb;
 }
 
-template <int DT, int QM, int KVM, int RM, bool MV>
+template <int DT, int QM, int KVM, int RM, bool MV, bool P2>
 hipError_t launch_one(DecodeParams p, int device, long long max_wg, long long cap, int cus, hipStream_t stream) {
     const size_t lds = (size_t)p.hpw * wave_lds<DT>() + (size_t)(p.nrows + 1) * sizeof(long long);
-    const void* kern = decode_kernel<DT, QM, KVM, RM, MV>();
+    const void* kern = decode_kernel<DT, QM, KVM, RM, MV, P2>();
     static std::atomic<unsigned long long> attr_done{0};
     const hipError_t ea = once_per_device(attr_done, device, [&] {
         // largest dynamic LDS any launch of this kernel asks for (4 waves, kMaxRows rows)
@@ -857,14 +862,14 @@ hipError_t launch_one(DecodeParams p, int device, long long max_wg, long long ca
     });
     if (ea != hipSuccess) return note_site(ea, "hipFuncSetAttribute(decode)");
     // one wave of workgroups that are all resident at once, bounded by the work
-    long long nwg = (long long)cus * resident_wgs<DT, QM, KVM, RM, MV>(p.hpw, lds);
+    long long nwg = (long long)cus * resident_wgs<DT, QM, KVM, RM, MV, P2>(p.hpw, lds);
     if (nwg > max_wg) nwg = max_wg;
     if (nwg > cap) nwg = cap;
     p.nwg = nwg < 1 ? 1 : (int)nwg;
     if constexpr (DT == kF32)
         hipLaunchKernelGGL((dv_decode<DT, QM, KVM, RM>), dim3(p.nwg), dim3(p.hpw * kWave), lds, stream, p);
     else
-        hipLaunchKernelGGL((dv_stream<DT, QM, KVM, RM, MV>), dim3(p.nwg), dim3(p.hpw * kWave), lds, stream, p);
+        hipLaunchKernelGGL((dv_stream<DT, QM, KVM, RM, MV, P2>), dim3(p.nwg), dim3(p.hpw * kWave), lds, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return note_site(e, "launch decode");
     const int nseg = p.nrows * (p.Hkv / p.hpw);
@@ -875,19 +880,25 @@ hipError_t launch_one(DecodeParams p, int device, long long max_wg, long long ca
     return hipSuccess;
 }
 
+template <int DT, int QM, int RM>
+hipError_t launch_paged(const DecodeParams& p, int device, long long max_wg, long long cap, int cus,
+                        hipStream_t stream) {
+    if constexpr (DT != kF32) {
+        if (p.F >= 2) return launch_one<DT, QM, kKvPaged, RM, true, false>(p, device, max_wg, cap, cus, stream);
+        if (p.bs_shift >= 4) return launch_one<DT, QM, kKvPaged, RM, false, true>(p, device, max_wg, cap, cus, stream);
+    }
+    return launch_one<DT, QM, kKvPaged, RM, false, false>(p, device, max_wg, cap, cus, stream);
+}
+
 template <int DT>
 hipError_t dispatch_modes(int qmode, int kvmode, int rowmode, const DecodeParams& p, int device, long long max_wg,
                           long long cap, int cus, hipStream_t stream) {
     if (kvmode == kKvPaged && qmode == kQRotFull && rowmode == kRowWS)
-        return p.F >= 2 && DT != kF32
-                   ? launch_one<DT, kQRotFull, kKvPaged, kRowWS, true>(p, device, max_wg, cap, cus, stream)
-                   : launch_one<DT, kQRotFull, kKvPaged, kRowWS, false>(p, device, max_wg, cap, cus, stream);
+        return launch_paged<DT, kQRotFull, kRowWS>(p, device, max_wg, cap, cus, stream);
     if (kvmode == kKvPaged && qmode == kQRotHalf && rowmode == kRowVarlen)
-        return p.F >= 2 && DT != kF32
-                   ? launch_one<DT, kQRotHalf, kKvPaged, kRowVarlen, true>(p, device, max_wg, cap, cus, stream)
-                   : launch_one<DT, kQRotHalf, kKvPaged, kRowVarlen, false>(p, device, max_wg, cap, cus, stream);
+        return launch_paged<DT, kQRotHalf, kRowVarlen>(p, device, max_wg, cap, cus, stream);
     if (kvmode == kKvContig && qmode == kQPre && rowmode == kRowWS)
-        return launch_one<DT, kQPre, kKvContig, kRowWS, false>(p, device, max_wg, cap, cus, stream);
+        return launch_one<DT, kQPre, kKvContig, kRowWS, false, false>(p, device, max_wg, cap, cus, stream);
     return hipErrorInvalidValue;
 }
 

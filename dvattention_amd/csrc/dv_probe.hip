@@ -41,7 +41,6 @@ __device__ unsigned read_piece(const DecodeParams& p, unsigned char* wlds, int r
     v.v = reinterpret_cast<const unsigned char*>(p.vc);
     v.off = 0;
     v.lp0 = 0;
-    v.a = 0;
     const int l0 = (int)v0, l1 = (int)(v1 < row_keys ? v1 : row_keys);
     const long long span = (long long)(stream::kPc - 1) * p.bs;
     for (int sa = l0; sa < l1;) {

@@ -511,7 +511,7 @@ struct View {
     const unsigned char* v;
     int off;                 // paged: logical position of the view's key 0
     int lp0;                 // paged: logical page of page-cache entry 0
-    int a, b;                // current view-local key range [a, b)
+    int b;                   // end (exclusive) of the current view-local key range
     int hkv;
 };
 
@@ -522,61 +522,85 @@ template <int KVM>
 __device__ inline uint32_t issue(const DecodeParams& p, const View& v, const int* pc, uint32_t sbase, int l) {
     const int lane = threadIdx.x & 63;
     const int c16 = lane & 15, sub = lane >> 4;
-    // addresses of the 8 key rows first (page-cache reads batched), then the loads
+    // addresses of the 8 key rows first (page-cache reads batched: unconditional,
+    // on a clamped index, as a branch around a read waits for it at once), then
+    // the loads.  Logical page and offset of a row (floor division: positions
+    // below 0 have pages below 0, which are not in the cache) step by four keys
+    // from the first row's, so a page size that is no power of two costs one
+    // division and not eight.
     const unsigned char* ka[8];
     const unsigned char* va[8];
     bool ok[8];
+    int lp = 0, r = 0, lp4 = 0, r4 = 0;
+    if (KVM == kKvPaged) {
+        const int pos = v.off + l + sub;
+        uint32_t q, x;
+        page_split(p, (uint32_t)(pos < 0 ? -1 - pos : pos), q, x);
+        lp = pos < 0 ? -1 - (int)q : (int)q;
+        r = pos < 0 ? p.bs - 1 - (int)x : (int)x;
+        page_split(p, 4u, q, x);
+        lp4 = (int)q;
+        r4 = (int)x;
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int kk = i * 4 + sub;
         const int key = l + kk;
         unsigned long long boff;
         if (KVM == kKvPaged) {
-            const int pos = v.off + key;
-            uint32_t lp, r;
-            page_split(p, pos > 0 ? (uint32_t)pos : 0u, lp, r);
-            const uint32_t idx = lp - (uint32_t)v.lp0;
-            const bool in = key >= v.a && key < v.b && pos >= 0 && idx < (uint32_t)kPc;
-            const int page = in ? pc[in ? idx : 0u] : -1;
-            ok[i] = page >= 0;
-            const uint32_t rowidx = ((uint32_t)page * (uint32_t)p.bs + r) * (uint32_t)p.Hkv + (uint32_t)v.hkv;
+            const uint32_t idx = (uint32_t)(lp - v.lp0);
+            const int page = pc[idx < (uint32_t)kPc ? idx : (uint32_t)(kPc - 1)];
+            ok[i] = key < v.b && idx < (uint32_t)kPc && page >= 0;
+            const uint32_t rowidx = ((uint32_t)page * (uint32_t)p.bs + (uint32_t)r) * (uint32_t)p.Hkv + (uint32_t)v.hkv;
             boff = (unsigned long long)rowidx << 8;
+            lp += lp4;
+            r += r4;
+            if (r >= p.bs) {
+                r -= p.bs;
+                ++lp;
+            }
         } else {
-            ok[i] = key >= v.a && key < v.b;
+            ok[i] = key < v.b;
             boff = (unsigned long long)(uint32_t)key << 8;
         }
         const int gk = c16 ^ (kk & 15), gv = c16 ^ ((kk & 7) << 1);
         ka[i] = ok[i] ? v.k + boff + gk * 16 : g_zero_row + gk * 16;
         va[i] = ok[i] ? v.v + boff + gv * 16 : g_zero_row + gv * 16;
     }
-    uint32_t mask = 0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         dma16(ka[i], sbase + (uint32_t)(i * 1024));
         dma16(va[i], sbase + (uint32_t)(kTile + i * 1024));
-        const uint64_t bl = ballot(ok[i]);
-        const uint32_t bits = (uint32_t)(bl & 1u) | (uint32_t)((bl >> 15) & 2u) | (uint32_t)((bl >> 30) & 4u) |
-                              (uint32_t)((bl >> 45) & 8u);
-        mask |= bits << (i * 4);
+    }
+    // the mask: the range's end, and, when some page of it is missing, the lanes'
+    // own verdicts bit by bit (rare; 60 scalar instructions)
+    const int nin = v.b - l;
+    uint32_t mask = nin >= kStep ? 0xffffffffu : (1u << (nin > 0 ? nin : 0)) - 1u;
+    if (KVM == kKvPaged) {
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) bad |= !ok[i] && ((mask >> (i * 4 + sub)) & 1u);
+        if (ballot(bad)) {
+            mask = 0;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint64_t bl = ballot(ok[i]);
+                const uint32_t bits = (uint32_t)(bl & 1u) | (uint32_t)((bl >> 15) & 2u) | (uint32_t)((bl >> 30) & 4u) |
+                                      (uint32_t)((bl >> 45) & 8u);
+                mask |= bits << (i * 4);
+            }
+        }
     }
     return mask;
 }
 
-// First key of the stages of a view whose range starts at key l0: paged stages
-// start at a multiple of 32 logical positions (possibly before the view; such
-// keys are invisible), so that with pages of a multiple of 16 keys each half of
-// a stage lies in one page.
-template <int KVM>
-__device__ inline int stage_start(int off, int l0) {
-    return KVM == kKvPaged ? l0 - ((off + l0) & (kStep - 1)) : l0;
-}
-
-// Whether the two pages (of 2^shift keys) of the stage at logical position pos,
-// a multiple of 16, have entries in the page cache, whose entry 0 is page lp0.
+// Whether a stage of 32 keys at logical position pos has two pages (of 2^shift
+// keys, shift >= 4), one for each half, with entries in the page cache, whose entry
+// 0 is page lp0.
 __host__ __device__ inline bool full_stage_in_cache(int pos, int shift, int lp0) {
     const uint32_t i0 = ((uint32_t)pos >> shift) - (uint32_t)lp0;
     const uint32_t i1 = (((uint32_t)pos + 16u) >> shift) - (uint32_t)lp0;
-    return pos >= 0 && i0 < (uint32_t)kPc && i1 < (uint32_t)kPc;
+    return pos >= 0 && (pos & 15) == 0 && i0 < (uint32_t)kPc && i1 < (uint32_t)kPc;
 }
 
 // This lane's byte offsets from the row base of a full stage's loads: load i
@@ -597,20 +621,22 @@ __device__ inline LaneOff lane_offsets(uint32_t row_stride) {
     return o;
 }
 
-// issue() of a paged stage that may be full: a stage whose 32 keys are all
-// visible, in pages of a power of two of at least 16 keys, needs no lane to look
-// up its rows: the two pages are read once for the wave, the row bases are scalar
-// and every load is a scalar base plus a lane constant -- about 120 instructions,
-// none of them vector arithmetic, where issue() takes 130 vector and 120 scalar
-// ones (one wave per SIMD: each is time the stage's loads and MFMAs wait for).
-// Everything but the lane offsets is wave-uniform.
-// A stage that reaches outside the page cache goes to issue(), which masks such
-// keys: positions below 0 (a negative fragment length before the view; lengths
-// are device data) have no entry.
+// issue() for calls of one view with pages of a power of two of at least 16 keys
+// (P2), whose stages start at multiples of 32 positions: a stage whose 32 keys are
+// all visible needs no lane to look up its rows: the two pages are read once for the
+// wave, the row bases are scalar and every load is a scalar base plus a lane
+// constant -- about 140 instructions, two of them vector arithmetic, where issue()
+// takes 210 vector and 130 scalar ones (one wave per SIMD: each is time the stage's
+// loads and MFMAs wait for).  Everything but the lane offsets is wave-uniform.  32
+// ragged sequences, pages of 16 keys: 97.9 us, 99.6 with issue() (pages of 24).
+// Calls of several views keep issue() alone: most of their stages start off a
+// multiple of 16, and a piece of short views pays for every path whose code it
+// fetches (16 rows of views of 700, 301, 93 and 41 keys: 25.2 us, 28.5 with both;
+// 4000, 3000, 2000 and 1000 keys: 64.9 / 64.3).
 __device__ inline uint32_t issue_stage(const DecodeParams& p, const View& v, const LaneOff& lo, const int* pc,
                                        uint32_t sbase, int l) {
     const int pos0 = v.off + l;
-    if (l >= v.a && l + kStep <= v.b && p.bs_shift >= 4 && full_stage_in_cache(pos0, p.bs_shift, v.lp0)) {
+    if (l + kStep <= v.b && full_stage_in_cache(pos0, p.bs_shift, v.lp0)) {
         const uint32_t pos = (uint32_t)pos0, in = (1u << p.bs_shift) - 1u;
         const int pg0 = uniform(pc[(int)(pos >> p.bs_shift) - v.lp0]);
         const int pg1 = uniform(pc[(int)((pos + 16) >> p.bs_shift) - v.lp0]);
@@ -632,13 +658,11 @@ __device__ inline uint32_t issue_stage(const DecodeParams& p, const View& v, con
     return (uint32_t)uniform((int)issue<kKvPaged>(p, v, pc, sbase, l));
 }
 
-// A stage of either kind.  Contiguous views keep the one general path: their
-// pieces end anywhere in a stage, and a short call pays for every path whose
-// code it fetches (four rows over 4.5k keys: 17.1 us with both, 15.6 with one).
-template <int KVM>
+// A stage of any kind.
+template <int KVM, bool P2>
 __device__ inline uint32_t issue_keys(const DecodeParams& p, const View& v, const LaneOff& lo, const int* pc,
                                       uint32_t sbase, int l) {
-    if constexpr (KVM == kKvPaged) return issue_stage(p, v, lo, pc, sbase, l);
+    if constexpr (P2) return issue_stage(p, v, lo, pc, sbase, l);
     else return issue<KVM>(p, v, pc, sbase, l);
 }
 

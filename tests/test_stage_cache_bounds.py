@@ -25,7 +25,7 @@ int main(int, char**) {
 
 def expected(pos, shift, lp0):
     pages = [(pos >> shift) - lp0, ((pos + 16) >> shift) - lp0]
-    return int(pos >= 0 and all(0 <= i < KPC for i in pages))
+    return int(pos >= 0 and pos % 16 == 0 and all(0 <= i < KPC for i in pages))
 
 
 def test_full_stage_in_cache(tmp_path):
@@ -41,7 +41,7 @@ def test_full_stage_in_cache(tmp_path):
         for lp0 in (0, 3, 1000):
             first = lp0 << shift
             for page in (-1, 0, 1, KPC - 2, KPC - 1, KPC):
-                cases += [(first + (page << shift) + o, shift, lp0) for o in (0, 16, (1 << shift) - 16)]
+                cases += [(first + (page << shift) + o, shift, lp0) for o in (0, 1, 8, 16, (1 << shift) - 16)]
             cases += [(p, shift, lp0) for p in (-16, -32, -64, -1 << 20, -1 << 31, (1 << 31) - 16, (1 << 31) - 32)]
     cases = [c for c in cases if -1 << 31 <= c[0] < 1 << 31]
     out = subprocess.run([str(exe)], input="\n".join("%d %d %d" % c for c in cases), capture_output=True, text=True,
