@@ -3,10 +3,10 @@
 //
 // Paged-read probe:
 // the 16-bit decode kernel's K/V stream with the attention taken out.  It runs
-// the decode's work split (run_schedule with the same start cost, XCD skew and
-// minimum range), fills the same per-wave page-id cache and streams every
-// visible K/V row of every piece through the same two-stage direct-to-LDS ring
-// (stream::issue) with the same completion waits -- but computes nothing: each
+// the decode's work split (run_schedule with the same start cost, XCD skew, minimum
+// range, grid and alignment of cuts), fills the same per-wave page-id cache and
+// streams every visible K/V row of every piece through the same two-stage
+// direct-to-LDS ring (stream::issue_keys) with the same completion waits -- but computes nothing: each
 // stage is consumed by one LDS word per lane.  Its rate is the HBM read rate
 // the decode's access pattern (256-byte rows of randomly placed pages) can
 // reach on the part, the ceiling the decode kernel is measured against.
@@ -27,6 +27,7 @@ namespace {
 
 // One wave: KV head hkv over visible keys [v0, v1) of a one-view row (the
 // decode's stream::piece minus the query, the MFMAs and the epilogue).
+template <bool P2>
 __device__ unsigned read_piece(const DecodeParams& p, unsigned char* wlds, int row, int hkv, long long v0,
                                long long v1, long long row_keys) {
     const int lane = threadIdx.x & 63;
@@ -41,8 +42,10 @@ __device__ unsigned read_piece(const DecodeParams& p, unsigned char* wlds, int r
     v.v = reinterpret_cast<const unsigned char*>(p.vc);
     v.off = 0;
     v.lp0 = 0;
+    const stream::LaneOff lo = stream::lane_offsets((uint32_t)p.Hkv << 8);
     const int l0 = (int)v0, l1 = (int)(v1 < row_keys ? v1 : row_keys);
-    const long long span = (long long)(stream::kPc - 1) * p.bs;
+    long long span = ((long long)(stream::kPc - 2) * p.bs) & ~(long long)(kStep - 1);
+    span = span < (1ll << 30) ? span : 1ll << 30;
     for (int sa = l0; sa < l1;) {
         const int sb = (long long)l1 - sa > span ? (int)(sa + span) : l1;
         v.b = sb;
@@ -50,25 +53,19 @@ __device__ unsigned read_piece(const DecodeParams& p, unsigned char* wlds, int r
         page_split(p, (uint32_t)sa, lpa, r);
         page_split(p, (uint32_t)(sb - 1), lpz, r);
         v.lp0 = (int)lpa;
-        const int need = (int)(lpz - lpa) + 1;
-        const int* bt = p.bt + (long long)w * p.maxB;
-        for (int i = lane; i < need; i += kWave) {
-            const uint32_t lp = lpa + (uint32_t)i;
-            int pg = lp < (uint32_t)p.maxB ? bt[lp] : -1;
-            if (pg < 0 || pg >= p.nblocks) pg = -1;
-            pc[i] = pg;
-        }
+        stream::fill_pages(p, p.bt + (long long)w * p.maxB, pc, (int)(lpz - lpa) + 1,
+                           [&](int i) { return lpa + (uint32_t)i; });
         const int n_st = (sb - sa + kStep - 1) / kStep;
-        uint32_t m = stream::issue<kKvPaged>(p, v, pc, ring, sa);
-        if (n_st > 1) m ^= stream::issue<kKvPaged>(p, v, pc, ring + stream::kStage, sa + kStep);
+        uint32_t m = stream::issue_keys<kKvPaged, P2>(p, v, lo, pc, ring, sa);
+        if (n_st > 1) m ^= stream::issue_keys<kKvPaged, P2>(p, v, lo, pc, ring + stream::kStage, sa + kStep);
         for (int s = 0; s < n_st; ++s) {
             if (s + 1 < n_st) wait_vmcnt<16>();
             else wait_vmcnt<0>();
             acc += *reinterpret_cast<const unsigned*>(wlds + (s & 1) * stream::kStage + lane * 4) ^ m;
             if (s + 2 < n_st) {
                 lds_wait();  // the slot's read is complete before it is refilled
-                m = stream::issue<kKvPaged>(p, v, pc, ring + (uint32_t)((s & 1) * stream::kStage),
-                                            sa + (s + 2) * kStep);
+                m = stream::issue_keys<kKvPaged, P2>(p, v, lo, pc, ring + (uint32_t)((s & 1) * stream::kStage),
+                                                     sa + (s + 2) * kStep);
             }
         }
         lds_wait();
@@ -77,18 +74,22 @@ __device__ unsigned read_piece(const DecodeParams& p, unsigned char* wlds, int r
     return acc;
 }
 
+template <bool P2>
 __global__ __launch_bounds__(256) void dv_read_probe(const DecodeParams p, unsigned* sink) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ long long s_scan[4];
-    const int wv = threadIdx.x >> 6;
+    const int wv = uniform((int)(threadIdx.x >> 6));
     const int HPW = p.hpw;
     long long* s_pref = reinterpret_cast<long long*>(smem + HPW * stream::kWaveLds);
     unsigned char* wlds = smem + wv * stream::kWaveLds;
     unsigned acc = 0;
-    run_schedule<true>(p, p.Hkv / HPW, s_pref, s_scan, [&](int row) { return row_visible<kKvPaged, kRowWS>(p, row); },
-                 [&](int row, int hg, long long v0, long long v1, bool, int, long long rk) {
-        if (wv < HPW) acc += read_piece(p, wlds, row, hg * HPW + wv, v0, v1, rk);
-    });
+    run_schedule<true, P2 ? kStep : 1>(
+        p, p.Hkv / HPW, s_pref, s_scan, [&](int row) { return row_visible<kKvPaged, kRowWS>(p, row); },
+        [&](int row, int hg, long long v0, long long v1, bool, int, long long rk) {
+            if (wv < HPW)
+                acc += read_piece<P2>(p, wlds, uniform(row), uniform(hg) * HPW + wv, uniform(v0), uniform(v1),
+                                      uniform(rk));
+        });
     if ((threadIdx.x & 63) == 0) sink[blockIdx.x * kMaxWavesPerWg + wv] = acc;
 }
 
@@ -266,34 +267,36 @@ __attribute__((visibility("default"))) int dvprobe_paged_read(int dtype, const i
     }
     p.dir = reinterpret_cast<int*>(workspace);
     const size_t lds = (size_t)p.hpw * stream::kWaveLds + (size_t)(p.nrows + 1) * sizeof(long long);
-    static std::atomic<unsigned long long> attr_done{0};
-    hipError_t e = once_per_device(attr_done, device, [&] {
+    const bool p2 = p.bs_shift >= 4;  // the decode's scalar stage path
+    const void* kern = p2 ? reinterpret_cast<const void*>(&dv_read_probe<true>)
+                          : reinterpret_cast<const void*>(&dv_read_probe<false>);
+    static std::atomic<unsigned long long> attr_done[2];
+    hipError_t e = once_per_device(attr_done[p2], device, [&] {
         const size_t max_lds = (size_t)kMaxWavesPerWg * stream::kWaveLds + (size_t)(kMaxRows + 1) * sizeof(long long);
-        return hipFuncSetAttribute(reinterpret_cast<const void*>(&dv_read_probe),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_lds);
+        return hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_lds);
     });
     if (e != hipSuccess) {
         g_msg = "probe: hipFuncSetAttribute failed";
         return -1;
     }
     int per_cu = 1;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(&dv_read_probe),
-                                                     p.hpw * kWave, lds) != hipSuccess || per_cu < 1)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, p.hpw * kWave, lds) != hipSuccess || per_cu < 1)
         per_cu = 1;
     // the decode's launch shape: one wave of resident workgroups, bounded by the work
     const int cus = device_cu_count(device);
     long long nwg = (long long)cus * per_cu;
     const long long max_wg = (long long)cus * (8 / p.hpw);
     if (nwg > max_wg) nwg = max_wg;
-    const long long cap = ((long long)p.nrows * nhg * s->max_blocks_per_seq * s->block_size + p.min_keys - 1) /
-                          p.min_keys;
+    const long long max_keys = (long long)s->max_blocks_per_seq * s->block_size;
+    const long long cap = ((long long)p.nrows * nhg * (max_keys + p.piece_cost) + p.min_keys - 1) / p.min_keys;
     if (nwg > cap) nwg = cap;
     p.nwg = nwg < 1 ? 1 : (int)nwg;
     if (sink_words < (long long)p.nwg * kMaxWavesPerWg || !sink) {
         g_msg = "probe: sink too small (4 words per workgroup)";
         return -1;
     }
-    hipLaunchKernelGGL(dv_read_probe, dim3(p.nwg), dim3(p.hpw * kWave), lds, (hipStream_t)stream, p, sink);
+    if (p2) hipLaunchKernelGGL(dv_read_probe<true>, dim3(p.nwg), dim3(p.hpw * kWave), lds, (hipStream_t)stream, p, sink);
+    else hipLaunchKernelGGL(dv_read_probe<false>, dim3(p.nwg), dim3(p.hpw * kWave), lds, (hipStream_t)stream, p, sink);
     if (hipGetLastError() != hipSuccess) {
         g_msg = "probe: launch failed";
         return -1;
