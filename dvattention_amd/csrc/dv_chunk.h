@@ -37,6 +37,14 @@ constexpr int kPieceCost = 256;
 // about 40 % less time there): 32 ragged sequences x 4 tokens, 1k - 8k keys, run
 // at 170 / 154 / 148.5 / 146.5 / 149 us with 128 / 256 / 400 / 512 / 768.
 constexpr int kPieceCostSplit = 512;
+// Varlen launches (row groups with and without the key split in one schedule): cost
+// units per key of a long group and of a short one (at most kFewTok tokens), so a
+// piece's start costs 256 and 512 of their keys, as above.  48 decodes beside two
+// prompt chunks, 4 KV heads (538 tokens, 256-8192 keys), with 3 : 8 / 1 : 2 /
+// 5 : 8 / 6 : 8: 174 / 160 / 168 / 176 us; prompts of 260-411 tokens, the last
+// groups short: 300 / 275 / 282 / 282.
+constexpr int kLongKeyCost = 2;
+constexpr int kShortKeyCost = 1;
 
 static __device__ __align__(16) unsigned char zrow[512];
 

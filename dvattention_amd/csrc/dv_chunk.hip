@@ -678,7 +678,9 @@ __device__ void chunk_piece(const DecodeParams& p, unsigned char* smem, int* pag
 }
 
 // P2: paged with a power-of-two block_size (shift and mask instead of a
-// division in the stage loop's row addressing).
+// division in the stage loop's row addressing).  KS = 0 (varlen): the key split of
+// each row group follows from its own tokens, four wave sets up to kFewTok tokens
+// and none above (decodes beside prompt chunks, and the last tokens of a chunk).
 template <int DT, int QM, int KVM, bool P2, int RM, int KS>
 __global__ __launch_bounds__(kThreads) void dv_chunk(const DecodeParams p) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -690,14 +692,34 @@ __global__ __launch_bounds__(kThreads) void dv_chunk(const DecodeParams p) {
     long long* s_pref = s_scan + kWaves;
     const int NHG = p.Hkv;  // one KV head per workgroup
 
-    // an empty list of groups (varlen): no cost to lay out, no piece
-    if (RM == kRowVarlen && blockIdx.x > 0 && p.vgroups[p.row_begin * 4 + 1] == 0) return;
-    run_schedule(p, NHG, s_pref, s_scan, [&](int rg) { return group_visible<KVM, RM>(p, rg); },
-                 [&](int rg, int hg, long long v0, long long v1, bool fin, int slot, long long rk) {
-                     chunk_piece<DT, QM, KVM, P2, RM, KS>(p, smem, pages, uniform(rg), uniform(hg), uniform(v0),
-                                                          uniform(v1), uniform((int)fin) != 0, uniform(slot),
-                                                          uniform(rk));
-                 });
+    if constexpr (KS > 0) {
+        run_schedule(p, NHG, s_pref, s_scan, [&](int rg) { return group_visible<KVM, RM>(p, rg); },
+                     [&](int rg, int hg, long long v0, long long v1, bool fin, int slot, long long rk) {
+                         chunk_piece<DT, QM, KVM, P2, RM, KS>(p, smem, pages, uniform(rg), uniform(hg), uniform(v0),
+                                                              uniform(v1), uniform((int)fin) != 0, uniform(slot),
+                                                              uniform(rk));
+                     });
+    } else {
+        // the schedule counts units (both sides of a cut round down alike); a split
+        // needs a positive scale (key_split)
+        auto unit = [&](int rg) {
+            return p.l2scale > 0.0f && group_of<RM>(p, rg).ntok <= kFewTok ? kShortKeyCost : kLongKeyCost;
+        };
+        run_schedule(p, NHG, s_pref, s_scan, [&](int rg) { return unit(rg) * group_visible<KVM, RM>(p, rg); },
+                     [&](int rg0, int hg, long long v0, long long v1, bool fin, int slot, long long rk) {
+                         const int rg = uniform(rg0);
+                         if (uniform(unit(rg)) == kShortKeyCost)
+                             chunk_piece<DT, QM, KVM, P2, RM, 4>(p, smem, pages, rg, uniform(hg),
+                                                                 uniform(v0 / kShortKeyCost),
+                                                                 uniform(v1 / kShortKeyCost), uniform((int)fin) != 0,
+                                                                 uniform(slot), uniform(rk / kShortKeyCost));
+                         else
+                             chunk_piece<DT, QM, KVM, P2, RM, 1>(p, smem, pages, rg, uniform(hg),
+                                                                 uniform(v0 / kLongKeyCost),
+                                                                 uniform(v1 / kLongKeyCost), uniform((int)fin) != 0,
+                                                                 uniform(slot), uniform(rk / kLongKeyCost));
+                     });
+    }
 }
 
 size_t lds_bytes(int nrows) {
@@ -712,13 +734,11 @@ size_t lds_bytes(int nrows) {
 // maximum of cu_seqlens_q[1 .. i + 1], sequence i's tokens are therefore
 // [max(0, M_{i-1}), min(T, M_i)) (M_{-1} = 0), and the tokens from M_{W-1} on
 // form one more run, of sequence 0 -- also for tables that are not
-// non-decreasing.  Each run is cut into groups of kTokBlk tokens; a last group of
-// at most `few` tokens goes to a list of its own, for a launch that splits the
-// keys (batches of decodes and prompt chunks: a decode's group would otherwise
-// be computed as 16 tokens).  One workgroup writes entry g = {first token,
-// tokens, sequence, 0} of every group of the two lists -- gmax entries for the
-// first, then W + 1 for the short groups (few > 0) -- and {0, 0, 0, 0} past each
-// list's end.  gmax is the host's bound (varlen_gmax).
+// non-decreasing.  Each run is cut into groups of kTokBlk tokens.  One
+// workgroup writes entry g = {first token, tokens, sequence, 0} for every
+// group, and {0, 0, 0, 0} for the entries from the group count up to gmax
+// (the host's bound T / kTokBlk + W + 1: a run of n tokens makes at most
+// n / kTokBlk + 1 groups).
 constexpr int kVgThreads = 1024;
 
 __device__ inline int block_scan_excl(int v, int* s_part, bool is_max) {
@@ -740,10 +760,9 @@ __device__ inline int block_scan_excl(int v, int* s_part, bool is_max) {
     return is_max ? (mine > before ? mine : before) : before + mine;
 }
 
-__global__ __launch_bounds__(kVgThreads) void dv_varlen_groups(const int* cu, int W, int T, int few, int gmax, int4* groups) {
+__global__ __launch_bounds__(kVgThreads) void dv_varlen_groups(const int* cu, int W, int T, int gmax, int4* groups) {
     __shared__ int s_m[kVarlenChunkMaxW];       // M_i
-    __shared__ int s_base[kVarlenChunkMaxW + 2];   // first group of run i (runs 0 .. W), then the total
-    __shared__ int s_sbase[kVarlenChunkMaxW + 2];  // the same for the short groups
+    __shared__ int s_base[kVarlenChunkMaxW + 2];  // first group of run i (runs 0 .. W), then the total
     __shared__ int s_part[kVgThreads / kWave];
     const int tid = threadIdx.x;
     // running maximum of cu[1 .. W], each thread over a contiguous block of sequences
@@ -765,60 +784,41 @@ __global__ __launch_bounds__(kVgThreads) void dv_varlen_groups(const int* cu, in
     };
     const int per1 = (W + 1 + kVgThreads - 1) / kVgThreads;
     const int j0 = tid * per1 < W + 1 ? tid * per1 : W + 1, j1 = j0 + per1 < W + 1 ? j0 + per1 : W + 1;
-    // groups of a run: {full or long ones, short ones}
-    auto count = [&](int i, int& c, int& sc) {
+    int cnt = 0;
+    for (int i = j0; i < j1; ++i) {
         int a, b;
         run(i, a, b);
-        const int n = b > a ? b - a : 0, rem = n % kTokBlk;
-        sc = rem > 0 && rem <= few ? 1 : 0;
-        c = n / kTokBlk + (rem > few ? 1 : 0);
-    };
-    int cnt = 0, scnt = 0;
-    for (int i = j0; i < j1; ++i) {
-        int c, sc;
-        count(i, c, sc);
+        const int c = b > a ? (b - a + kTokBlk - 1) / kTokBlk : 0;
+        s_base[i] = c;
         cnt += c;
-        scnt += sc;
     }
     int acc = block_scan_excl(cnt, s_part, false);
-    __syncthreads();
-    int sacc = block_scan_excl(scnt, s_part, false);
     for (int i = j0; i < j1; ++i) {
-        int c, sc;
-        count(i, c, sc);
+        const int c = s_base[i];
         s_base[i] = acc;
-        s_sbase[i] = sacc;
         acc += c;
-        sacc += sc;
     }
-    if (tid == kVgThreads - 1) {
-        s_base[W + 1] = acc;
-        s_sbase[W + 1] = sacc;
-    }
+    if (tid == kVgThreads - 1) s_base[W + 1] = acc;
     __syncthreads();
-    const int total = s_base[W + 1], stotal = s_sbase[W + 1];
-    const int entries = gmax + (few > 0 ? W + 1 : 0);
-    for (int e0 = tid; e0 < entries; e0 += kVgThreads) {
+    const int total = s_base[W + 1];
+    for (int gi = tid; gi < gmax; gi += kVgThreads) {
         int4 e = {0, 0, 0, 0};
-        const bool is_short = e0 >= gmax;
-        const int gi = is_short ? e0 - gmax : e0;
-        const int* base = is_short ? s_sbase : s_base;
-        if (gi < (is_short ? stotal : total)) {
+        if (gi < total) {
             // the last run whose first group is <= gi (it has groups: the next run's first is larger)
             int lo = 0, hi = W;
             while (lo < hi) {
                 const int mid = (lo + hi + 1) >> 1;
-                if (base[mid] <= gi) lo = mid;
+                if (s_base[mid] <= gi) lo = mid;
                 else hi = mid - 1;
             }
             int a, b;
             run(lo, a, b);
-            const int t0 = a + (is_short ? (b - a) / kTokBlk : gi - base[lo]) * kTokBlk;
+            const int t0 = a + (gi - s_base[lo]) * kTokBlk;
             e.x = t0;
             e.y = b - t0 < kTokBlk ? b - t0 : kTokBlk;
             e.z = lo == W ? 0 : lo;
         }
-        groups[e0] = e;
+        groups[gi] = e;
     }
 }
 
@@ -837,18 +837,20 @@ hipError_t launch1(DecodeParams p, int device, int cus, long long cap, hipStream
     hipLaunchKernelGGL((dv_chunk<DT, QM, KVM, P2, RM, KS>), dim3(p.nwg), dim3(kThreads), lds, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    int ntb = max_group_tokens<RM>(p);
-    if (KS == 4 && ntb > kFewTok) ntb = kFewTok;
+    const int ntb = max_group_tokens<RM>(p);
     hipLaunchKernelGGL((dv_merge_chunk<DT, RM>), dim3(p.nrows * p.Hkv * ntb), dim3(256), 0, stream, p, ntb);
     return hipGetLastError();
 }
 
 template <int DT, int QM, int KVM, int RM, bool P2>
 hipError_t launch_split(const DecodeParams& p, int ks, int device, int cus, long long cap, hipStream_t stream) {
-    if (ks == 4) return launch1<DT, QM, KVM, P2, RM, 4>(p, device, cus, cap, stream);
-    if constexpr (RM != kRowVarlen)  // varlen launches: groups of at most kFewTok tokens, or any
+    if constexpr (RM == kRowVarlen) {
+        return launch1<DT, QM, KVM, P2, RM, 0>(p, device, cus, cap, stream);
+    } else {
+        if (ks == 4) return launch1<DT, QM, KVM, P2, RM, 4>(p, device, cus, cap, stream);
         if (ks == 2) return launch1<DT, QM, KVM, P2, RM, 2>(p, device, cus, cap, stream);
-    return launch1<DT, QM, KVM, P2, RM, 1>(p, device, cus, cap, stream);
+        return launch1<DT, QM, KVM, P2, RM, 1>(p, device, cus, cap, stream);
+    }
 }
 
 template <int DT, int QM, int KVM, int RM>
@@ -865,8 +867,12 @@ hipError_t launch(const DecodeParams& p, int ks, int device, int cus, long long 
 // Key split of a launch whose groups have at most ntok tokens: as many wave sets
 // as hold two tokens per wave.  (Eight sets for two tokens would take a ring step
 // of all eight stages, with nothing in flight beside it; two tokens run at 5.3
-// TB/s with four.)  A split step with no visible key must leave no trace in the
-// softmax, which -inf scores only do for a positive scale.
+// TB/s with four.)  Faster than no split over the whole range: 2 / 4 / 8 tokens,
+// bf16, one sequence of 3001 keys, 8 KV heads 29.7 / 30.8 / 32.7 -> 26.2 / 27.1 /
+// 29.1 us; fp16, 32 x 4608 keys 224 / 223 / 234 -> 112 / 114 / 153; contiguous fp16,
+// 16 x 4096 keys 119 / 120 / 122 -> 60 / 63 / 84; 64 x 60-100 keys, bf16 50.1 /
+// 52.5 / 58.7 -> 45.1 / 47.0 / 51.6.  A split step with no visible key must leave no
+// trace in the softmax, which -inf scores only do for a positive scale.
 int key_split(float l2scale, int ntok) {
     if (!(l2scale > 0.0f) || ntok > 8) return 1;
     return ntok > kFewTok ? 2 : 4;
@@ -890,23 +896,12 @@ ChunkWs chunk_ws(long long groups, int Hkv, int device, bool varlen) {
     ChunkWs l;
     l.part = ((size_t)((chunk_cus(device) + nseg) * slot_floats * 4) + 255) & ~(size_t)255;
     l.dir = ((size_t)(nseg * 2 * 4) + 255) & ~(size_t)255;
-    l.vgroups = varlen ? (size_t)groups * 2 * 16 : 0;  // two lists (dv_varlen_groups)
+    l.vgroups = varlen ? (size_t)groups * 16 : 0;
     l.total = l.part + l.dir + l.vgroups;
     return l;
 }
 
-// Groups of a varlen call at most: a run of n tokens makes n / kTokBlk of
-// kTokBlk tokens and one more, and there are W + 1 runs; with short groups listed
-// apart, the others have more than kFewTok tokens.
-long long varlen_gmax(int T, int W, bool few) {
-    const long long g = (long long)T / chunk::kTokBlk + W + 1;
-    const long long n = T / (chunk::kFewTok + 1);
-    return few && n < g ? n : g;
-}
-
-// Keys (of all sequences and KV heads) from which a varlen call lists its short
-// groups apart.
-constexpr long long kFewMinKeys = 1ll << 18;
+long long varlen_gmax(int T, int W) { return (long long)T / chunk::kTokBlk + W + 1; }
 
 // The chunk launches over `groups` row groups, kMaxRows at a time.
 template <int RM>
@@ -921,7 +916,11 @@ hipError_t launch_groups(int dtype, int qmode, int kvmode, DecodeParams p, long 
     p.slot_floats = chunk::kTokBlk * kGqa * (kHeadDim + 1);
     p.part = reinterpret_cast<float*>(workspace);
     p.dir = reinterpret_cast<int*>(reinterpret_cast<unsigned char*>(workspace) + l.part);
-    p.piece_cost = ks == 1 ? chunk::kPieceCost : chunk::kPieceCostSplit;
+    // ks = 0: the schedule counts in cost units (dv_chunk)
+    const int unit = ks == 0 ? chunk::kLongKeyCost : 1;
+    p.piece_cost = unit * (ks <= 1 ? chunk::kPieceCost : chunk::kPieceCostSplit);
+    const int min_keys = p.min_keys;
+    p.min_keys *= unit;
     // odd workgroups (odd XCD of each pair) take shorter chunks, as in the decode
     // split; 30 per mille measured best on configuration 5
     static const int skew = env_per_mille("DVATTN_CHUNK_SKEW_PM", 30);
@@ -929,7 +928,7 @@ hipError_t launch_groups(int dtype, int qmode, int kvmode, DecodeParams p, long 
     for (long long g0 = 0; g0 < groups_total; g0 += kMaxRows) {
         p.row_begin = (int)g0;
         p.nrows = (int)(groups_total - g0 < kMaxRows ? groups_total - g0 : kMaxRows);
-        const long long cap = ((long long)p.nrows * p.Hkv * max_keys_per_group + p.min_keys - 1) / p.min_keys;
+        const long long cap = ((long long)p.nrows * p.Hkv * max_keys_per_group + min_keys - 1) / min_keys;
         if constexpr (RM == kRowVarlen) {
             if (dtype == kBF16 && qmode == kQRotHalf && kvmode == kKvPaged)
                 e = chunk::launch<kBF16, kQRotHalf, kKvPaged, RM>(p, ks, device, cus, cap, stream);
@@ -982,7 +981,7 @@ hipError_t launch_chunk(int dtype, int qmode, int kvmode, const DecodeParams& ba
 
 size_t varlen_chunk_workspace_bytes(int T, int W, int Hkv, int device) {
     if (T <= 0 || W <= 0 || Hkv <= 0) return 0;
-    return chunk_ws(varlen_gmax(T, W, false), Hkv, device, true).total;
+    return chunk_ws(varlen_gmax(T, W), Hkv, device, true).total;
 }
 
 hipError_t launch_varlen_chunk(int dtype, const DecodeParams& base, long long max_keys_per_group, void* workspace,
@@ -992,39 +991,19 @@ hipError_t launch_varlen_chunk(int dtype, const DecodeParams& base, long long ma
     int device = 0;
     hipError_t e = hipGetDevice(&device);
     if (e != hipSuccess) return e;
-    const ChunkWs l = chunk_ws(varlen_gmax(base.T, base.W, false), base.Hkv, device, true);
+    const long long gmax = varlen_gmax(base.T, base.W);
+    const ChunkWs l = chunk_ws(gmax, base.Hkv, device, true);
     if (ws_bytes < l.total) return hipErrorInvalidValue;
-    // the decodes of a mixed batch apart from its chunks (16-bit types; a key
-    // split needs a positive scale), where the sequences' keys are worth the
-    // second launch and merge: those cost 5 us of a call without short groups
-    // (2 x 64 tokens, 500 keys, 8 KV heads: 43.5 -> 48.3 us; 4 x 4 x 500: 31.4 ->
-    // 36.8), the split saves a quarter of a call of short ones (32 x 4 x 4608
-    // keys: 185 -> 124 us)
-    // T a multiple of W: taken for a uniform batch, which has short groups only if
-    // its token count per sequence ends in one (16 x 16 tokens, 8208 keys: 179 us
-    // with one launch, 184-190 with an empty second one)
-    const int rem = base.T / base.W % chunk::kTokBlk;
-    const bool no_short = base.T % base.W == 0 && (rem == 0 || rem > chunk::kFewTok);
-    const int ks = dtype == kF32 || no_short || base.W * (long long)base.Hkv * max_keys_per_group < kFewMinKeys
-                       ? 1
-                       : chunk::key_split(base.l2scale, chunk::kFewTok);
-    const int few = ks > 1 ? chunk::kFewTok : 0;
-    const long long gmax = varlen_gmax(base.T, base.W, few > 0);
     DecodeParams p = base;
     int4* groups = reinterpret_cast<int4*>(reinterpret_cast<unsigned char*>(workspace) + l.part + l.dir);
+    p.vgroups = reinterpret_cast<const int*>(groups);
     hipLaunchKernelGGL(chunk::dv_varlen_groups, dim3(1), dim3(chunk::kVgThreads), 0, stream, base.cu_q, base.W,
-                       base.T, few, (int)gmax, groups);
+                       base.T, (int)gmax, groups);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    // one launch after the other on the same partial slots
-    if (few > 0) {
-        p.vgroups = reinterpret_cast<const int*>(groups + gmax);
-        e = launch_groups<kRowVarlen>(dtype, kQRotHalf, kKvPaged, p, base.W + 1, max_keys_per_group, ks, l, workspace,
-                                      stream);
-        if (e != hipSuccess || gmax == 0) return e;
-    }
-    p.vgroups = reinterpret_cast<const int*>(groups);
-    return launch_groups<kRowVarlen>(dtype, kQRotHalf, kKvPaged, p, gmax, max_keys_per_group, 1, l, workspace, stream);
+    const int ks = dtype == kF32 ? 1 : 0;
+    return launch_groups<kRowVarlen>(dtype, kQRotHalf, kKvPaged, p, gmax, max_keys_per_group, ks, l, workspace,
+                                     stream);
 }
 
 }  // namespace dv

@@ -40,14 +40,16 @@ def test_contiguous_few_tokens(dv, gpu, S):  # noqa: F811
     close(out, O.contig_sdpa(0.1, loc, q, fl, ks, vs), torch.bfloat16, f"S={S}")
 
 
-# tokens per sequence: groups of 4 or fewer are listed apart from longer ones
+# tokens per sequence: groups of 4 or fewer split their keys, longer ones in the same
+# launch do not; pages that are and are not a power of two, pieces cut inside groups
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bs", [16, 24])
 @pytest.mark.parametrize("counts,lens", [
     ([1, 1, 40, 1, 3], [700]), ([4, 5, 16, 17, 20, 21, 0, 1], [90, 40]), ([2, 2], [50]), ([16, 32], [300]),
-    ([1] * 6 + [30], [2000, 33, 0])])
-def test_varlen_mixed_groups(dv, gpu, dtype, counts, lens):  # noqa: F811
+    ([4] * 4, [600]), ([1, 1, 1, 29], [500]), ([1, 3], [9000]), ([3, 36], [5000]), ([1] * 6 + [30], [2000, 33, 0])])
+def test_varlen_mixed_groups(dv, gpu, dtype, bs, counts, lens):  # noqa: F811
     W, T = len(counts), sum(counts)
-    d = rand_varlen(len(lens), W, T, np.concatenate([[0], np.cumsum(counts)]), 2, 16, lens, 64, dtype, seed=T)
+    d = rand_varlen(len(lens), W, T, np.concatenate([[0], np.cumsum(counts)]), 2, bs, lens, 64, dtype, seed=T)
     close(run_varlen(dv, d, 0.1, gpu), O.varlen_paged_sdpa(0.1, **d), dtype, f"{counts}")
 
 
