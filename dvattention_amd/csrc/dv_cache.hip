@@ -190,23 +190,36 @@ __global__ __launch_bounds__(256) void dv_view_meta(const MetaParams p, long lon
     // the whole row is walked: if f appears more than once, its first place
     // wins, as in the reference, whose backward walk assigns it last.  The row is
     // walked eight segments at a time, their loads issued together (one after the
-    // other, a row of five segments was ten dependent round trips)
+    // other, a row of five segments was ten dependent round trips: 20 calls on 5 / 8
+    // / 16 / 40 segments 64 / 73 / 98 / 182 us, batched 60 / 62 / 75 / 133); rows of
+    // up to three one by one (one segment: 47 us, batched 50)
     long long suffix = 0, at = 0;
     bool found = false;
     const int* ord = p.order + (long long)w * p.F;
-    for (int j0 = p.F - 1; j0 >= 0; j0 -= 8) {
-        int g[8], len[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) g[k] = ord[j0 - k > 0 ? j0 - k : 0];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) len[k] = p.fl[g[k] >= 0 && g[k] < p.F ? g[k] : 0];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (j0 - k < 0) continue;
-            if (g[k] >= 0 && g[k] < p.F) suffix += len[k];
-            if (g[k] == f) {
+    if (p.F <= 3) {
+        for (int j = p.F - 1; j >= 0; --j) {
+            const int g = ord[j];
+            if (g >= 0 && g < p.F) suffix += p.fl[g];
+            if (g == f) {
                 found = true;
                 at = suffix;
+            }
+        }
+    } else {
+        for (int j0 = p.F - 1; j0 >= 0; j0 -= 8) {
+            int g[8], len[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) g[k] = ord[j0 - k > 0 ? j0 - k : 0];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) len[k] = p.fl[g[k] >= 0 && g[k] < p.F ? g[k] : 0];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                if (j0 - k < 0) continue;
+                if (g[k] >= 0 && g[k] < p.F) suffix += len[k];
+                if (g[k] == f) {
+                    found = true;
+                    at = suffix;
+                }
             }
         }
     }
