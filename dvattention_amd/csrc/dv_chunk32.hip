@@ -259,10 +259,10 @@ __device__ void chunk32_piece(const DecodeParams& p, unsigned char* smem, int* p
                 r.b = sbnd;
                 r.pages_ok = true;
                 if (KVM == kKvPaged) {
-                    r.lp0 = logical_page(p, off + sa);
+                    r.lp0 = uniform((int)logical_page(p, off + sa));
                     __syncthreads();  // every wave is done with the previous sub-range's page ids
                     static_assert(kWaves32 * kWave == kThreads, "one page-cache fill per workgroup");
-                    const uint32_t lpl = logical_page(p, off + sbnd - 1);
+                    const uint32_t lpl = uniform((int)logical_page(p, off + sbnd - 1));
                     int pg[kPageIt];
                     fetch_pages(p, p.bt + (long long)w * p.maxB, r.lp0, lpl, pg);
                     store_pages(p, pages, r.lp0, lpl, pg);
