@@ -605,8 +605,6 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
                                [&](int i) { return lpa + (uint32_t)i; });
                 }
                 const int n_st = (sb - sa + kStep - 1) / kStep;
-                // the first two stages in a rolled loop: this code runs once per piece,
-                // and a second copy of it would be fetched cold
                 // the first two stages; a contiguous call's in a rolled loop (its code runs
                 // once per piece, and a second copy of it would be fetched cold: 16 rows
                 // of 2000 keys 33.0 us, 33.4 with two copies), which costs paged calls
@@ -666,9 +664,11 @@ __device__ void piece(const DecodeParams& p, unsigned char* wlds, int row, int h
                      uniform(__shfl(t.off, f, kWave)));
         }
     } else if (v0 < v1) {
-        for_views<KVM, RM>(p, row, v0, v1, [&](int f, int vis, long long P, long long off) {
+        auto body = [&](int f, int vis, long long P, long long off) {
             one_view(f, uniform(vis), uniform(P), uniform(off));
-        });
+        };
+        if constexpr (P2) for_views<KVM, RM>(p, row, v0, v1, body);  // one view: never reached
+        else for_views_blocks<KVM, RM>(p, row, v0, v1, body);
     }
 
     // epilogue: total over the four lane groups, normalise, base-2 LSE

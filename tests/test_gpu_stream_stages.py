@@ -40,3 +40,20 @@ def test_invalid_page_in_a_full_stage(dv, gpu, bs):  # noqa: F811
     k = d["k_cache"][pages, pos % bs, 0].float()
     v = d["v_cache"][pages, pos % bs, 0].float()
     close(out[0, :, 0], torch.softmax(0.1 * (rq @ k.T), -1) @ v, torch.bfloat16, f"bs={bs}")
+
+
+# rows of more than 64 views, whose table is walked 64 at a time: one view more than a
+# block, two blocks, views without keys (some of them unseen by their query), page
+# positions past the first block
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("F,bs", [(64, 16), (65, 16), (129, 24), (140, 32)])
+def test_paged_many_views(dv, gpu, dtype, F, bs):  # noqa: F811
+    rng = np.random.default_rng(F)
+    lens = rng.integers(0, 90, size=F)
+    lens[[0, 63, -1]] = [70, 33, 41]
+    loc = rng.integers(-1, 90, size=(F, 3, 1))
+    d = rand_paged(F, 3, 1, 4, bs, list(lens), 32, dtype, seed=bs, loc=loc)
+    close(run_paged(dv, d, 0.1, gpu), O.paged_sdpa(0.1, **d), dtype, f"F={F}")
+    loc[64:] = -1  # no view of the later blocks is seen
+    d = rand_paged(F, 3, 1, 4, bs, list(lens), 32, dtype, seed=bs, loc=loc)
+    close(run_paged(dv, d, 0.1, gpu), O.paged_sdpa(0.1, **d), dtype, f"F={F}, first block only")
