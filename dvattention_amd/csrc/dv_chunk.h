@@ -45,6 +45,9 @@ constexpr int kPieceCostSplit = 512;
 // groups short: 300 / 275 / 282 / 282.
 constexpr int kLongKeyCost = 2;
 constexpr int kShortKeyCost = 1;
+// Keys per view from which a launch of few tokens per sequence splits them (key_split).
+constexpr int kSplitMinKeys = 48;
+constexpr int kSplitContig2Keys = 128;
 
 static __device__ __align__(16) unsigned char zrow[512];
 

@@ -401,10 +401,18 @@ __device__ inline void stream_range(const DecodeParams& p, const Range& r, const
     const uint32_t ring = lds_addr(smem);
     const int nsteps = (sbnd - sa + KS * kStep - 1) / (KS * kStep);
     const float l2 = p.l2scale;
-    // prologue: steps 0 .. kLead-1 (past the end: rows of zeros)
+    // prologue: steps 0 .. kLead-1.  Past the end, KS = 1 issues rows of zeros; with a
+    // key split such steps issue nothing (a view of 30 keys would pay for the
+    // addresses of 12 stages and not 4: 2 tokens, 4 sequences, six such views, 8 KV
+    // heads 112.5 -> 99.6 us; six of 150 keys 55 -> 50.5).
 #pragma unroll
-    for (int st = 0; st < kLead * KS; ++st) issue_stage<KVM, P2>(p, r, pages, ring, st, sa + st * kStep);
-    wait_vmcnt<kDma * (kLead - 1)>();  // own share of step 0 landed
+    for (int s = 0; s < kLead; ++s) {
+        if (KS > 1 && s >= nsteps) break;
+#pragma unroll
+        for (int st = s * KS; st < (s + 1) * KS; ++st) issue_stage<KVM, P2>(p, r, pages, ring, st, sa + st * kStep);
+    }
+    if (KS == 1 || nsteps >= kLead) wait_vmcnt<kDma * (kLead - 1)>();  // own share of step 0 landed
+    else wait_vmcnt<0>();
     wg_barrier();
 
     KOp kop;
@@ -445,9 +453,12 @@ __device__ inline void stream_range(const DecodeParams& p, const Range& r, const
         }
         settle<DT>(pa);
         lds_wait();
-        wait_vmcnt<kDma * (kLead - 2)>();  // own share of step i + 1 landed
+        // own share of step i + 1 landed (with a key split, fewer loads follow it near
+        // the end)
+        if (KS == 1 || i + kLead <= nsteps) wait_vmcnt<kDma * (kLead - 2)>();
+        else wait_vmcnt<0>();
         wg_barrier();
-        if constexpr (KS > 1) {
+        if (KS > 1 && i + kLead < nsteps) {
             // the loads of step i + kLead, into the slots of step i (free since the
             // barrier): at once, as no later step is in flight when KS = 4; one
             // stage at a time, the addresses of all do not fit the registers
@@ -455,8 +466,9 @@ __device__ inline void stream_range(const DecodeParams& p, const Range& r, const
             for (int q = (i + kLead) * KS; q < (i + kLead + 1) * KS; ++q)
                 issue_stage<KVM, P2>(p, r, pages, ring, q, sa + q * kStep);
         }
-        // ---- H2(i) (step i + 1 has landed even past the end -- rows of zeros --
-        // so K and S_A of the next stage need no branch; the last ones go unused)
+        // ---- H2(i) (past the end, step i + 1 holds rows of zeros or what the slot
+        // held before: K and S_A of the next stage need no branch, the last ones go
+        // unused)
         read_k(smem + ((st + KS) % kStages) * kStageBytes, kop);
         if (mkb != 0xffffffffu) mask_scores(sb0, sb1, mkb);
         mfma_settle(tl[1].o);
@@ -872,10 +884,18 @@ hipError_t launch(const DecodeParams& p, int ks, int device, int cus, long long 
 // 29.1 us; fp16, 32 x 4608 keys 224 / 223 / 234 -> 112 / 114 / 153; contiguous fp16,
 // 16 x 4096 keys 119 / 120 / 122 -> 60 / 63 / 84; 64 x 60-100 keys, bf16 50.1 /
 // 52.5 / 58.7 -> 45.1 / 47.0 / 51.6.  A split step with no visible key must leave no
-// trace in the softmax, which -inf scores only do for a positive scale.
-int key_split(float l2scale, int ntok) {
+// trace in the softmax, which -inf scores only do for a positive scale.  Short views
+// gain nothing (each one's queries are staged for all sets, and a piece ends with the
+// sets' combination), so a call is split from 48 keys per view on, as far as the host
+// knows them (paged: what the block tables hold), and a contiguous one of 5 - 8
+// tokens in several views from 128 on: without the split / with it, 8 KV heads, 6 x 30
+// contiguous keys, 2 tokens 68 / 76 us, paged 96 / 99; 12 x 90 contiguous, 8 tokens 62
+// / 67; 6 x 60 paged, 2 / 8 tokens 65 / 62, 70 / 62; 6 x 150 contiguous, 8 tokens 51 / 50.
+int key_split(float l2scale, int ntok, long long keys, int F, bool contig) {
     if (!(l2scale > 0.0f) || ntok > 8) return 1;
-    return ntok > kFewTok ? 2 : 4;
+    const int ks = ntok > kFewTok ? 2 : 4;
+    const long long per_view = contig && ks == 2 && F > 1 ? kSplitContig2Keys : kSplitMinKeys;
+    return keys < per_view * F ? 1 : ks;
 }
 
 }  // namespace chunk
@@ -975,7 +995,9 @@ hipError_t launch_chunk(int dtype, int qmode, int kvmode, const DecodeParams& ba
     const long long groups = (long long)base.W * ((base.S + chunk::kTokBlk - 1) / chunk::kTokBlk);
     const ChunkWs l = chunk_ws(groups, base.Hkv, device, false);
     if (ws_bytes < l.total) return hipErrorInvalidValue;
-    const int ks = dtype == kF32 ? 1 : chunk::key_split(base.l2scale, base.S);
+    const int ks = dtype == kF32 ? 1
+                                 : chunk::key_split(base.l2scale, base.S, max_keys_per_group, base.F,
+                                                    kvmode == kKvContig);
     return launch_groups<kRowWS>(dtype, qmode, kvmode, base, groups, max_keys_per_group, ks, l, workspace, stream);
 }
 

@@ -53,6 +53,24 @@ def test_varlen_mixed_groups(dv, gpu, dtype, bs, counts, lens):  # noqa: F811
     close(run_varlen(dv, d, 0.1, gpu), O.varlen_paged_sdpa(0.1, **d), dtype, f"{counts}")
 
 
+# views of one, two and more steps of a split (its loads end with the last step), and
+# contiguous views below and above the length from which 5 - 8 tokens are split
+@pytest.mark.parametrize("S", [3, 7])
+@pytest.mark.parametrize("lens", [[47], [48, 48], [129, 63, 65], [128, 128, 128, 256], [600, 385, 17]])
+def test_split_steps(dv, gpu, S, lens):  # noqa: F811
+    F, W, Hkv, dtype = len(lens), 2, 2, torch.bfloat16
+    loc = np.array(lens)[:, None, None] - S + np.arange(S) + np.zeros((F, W, 1), int)
+    d = rand_paged(F, W, S, Hkv, 16, lens, 64, dtype, seed=S + sum(lens), loc=loc)
+    close(run_paged(dv, d, 0.1, gpu), O.paged_sdpa(0.1, **d), dtype, f"paged S={S} {lens}")
+    g = torch.Generator().manual_seed(S)
+    q = torch.randn(F, W, 16 * Hkv, S, 128, generator=g).to(dtype)
+    ks = [torch.randn(W, Hkv, L, 128, generator=g).to(dtype) for L in lens]
+    vs = [torch.randn(W, Hkv, L, 128, generator=g).to(dtype) for L in lens]
+    fl, lc = torch.tensor(lens, dtype=torch.int32), torch.from_numpy(loc.astype(np.int32))
+    out = dv.dvattn_sdpa(q.to(gpu), lc.to(gpu), [k.to(gpu) for k in ks], [v.to(gpu) for v in vs], 0.1, fl.to(gpu))
+    close(out, O.contig_sdpa(0.1, lc, q, fl, ks, vs), dtype, f"contiguous S={S} {lens}")
+
+
 def test_varlen_mixed_unsorted_table(dv, gpu):  # noqa: F811
     # a table that is not non-decreasing, and tokens past its last entry
     d = rand_varlen(2, 4, 45, np.array([0, 3, 2, 30, 29]), 1, 16, [60, 200], 32, torch.bfloat16, seed=5)
