@@ -38,14 +38,18 @@ constexpr int kPieceCost = 256;
 // at 170 / 154 / 148.5 / 146.5 / 149 us with 128 / 256 / 400 / 512 / 768.
 constexpr int kPieceCostSplit = 512;
 // Varlen launches (row groups with and without the key split in one schedule): cost
-// units per key of a long group and of a short one (at most kFewTok tokens), so a
-// piece's start costs 256 and 512 of their keys, as above.  48 decodes beside two
-// prompt chunks, 4 KV heads (538 tokens, 256-8192 keys), with 3 : 8 / 1 : 2 /
-// 5 : 8 / 6 : 8: 174 / 160 / 168 / 176 us; prompts of 260-411 tokens, the last
-// groups short: 300 / 275 / 282 / 282.
-constexpr int kLongKeyCost = 2;
-constexpr int kShortKeyCost = 1;
-// Keys per view from which a launch of few tokens per sequence splits them (key_split).
+// units per key of a long group and of a split one, so a piece's start costs 256 and
+// 512 of their keys, as above.  48 decodes beside two prompt chunks, 4 KV heads (538
+// tokens, 256-8192 keys), with 3 : 8 / 1 : 2 / 5 : 8 / 6 : 8: 174 / 160 / 168 / 176
+// us; prompts of 260-411 tokens, the last groups short: 300 / 275 / 282 / 282.  Even
+// numbers, as a cost's lowest bit says which kind the group is (dv_chunk).
+constexpr int kLongKeyCost = 4;
+constexpr int kShortKeyCost = 2;
+// Keys per view from which a varlen launch splits a group of at most kFewTok tokens.
+// Block tables of 2048 pages, 20 x 2 + 16 tokens, 20 / 40 / 80 / 100 keys, 8 KV heads:
+// 26.8 / 28.4 / 30.1 / 32.0 us without the split, 32.7 / 33.0 / 33.7 / 30.0 with it.
+constexpr int kSplitVarlenKeys = 96;
+// The same for a launch of few tokens per sequence (key_split).
 constexpr int kSplitMinKeys = 48;
 constexpr int kSplitContig2Keys = 128;
 

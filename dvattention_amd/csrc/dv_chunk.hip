@@ -712,21 +712,25 @@ __global__ __launch_bounds__(kThreads) void dv_chunk(const DecodeParams p) {
                                                               uniform(rk));
                      });
     } else {
-        // the schedule counts units (both sides of a cut round down alike); a split
-        // needs a positive scale (key_split)
-        auto unit = [&](int rg) {
-            return p.l2scale > 0.0f && group_of<RM>(p, rg).ntok <= kFewTok ? kShortKeyCost : kLongKeyCost;
-        };
-        run_schedule(p, NHG, s_pref, s_scan, [&](int rg) { return unit(rg) * group_visible<KVM, RM>(p, rg); },
-                     [&](int rg0, int hg, long long v0, long long v1, bool fin, int slot, long long rk) {
-                         const int rg = uniform(rg0);
-                         if (uniform(unit(rg)) == kShortKeyCost)
-                             chunk_piece<DT, QM, KVM, P2, RM, 4>(p, smem, pages, rg, uniform(hg),
+        // the schedule counts units, even for a group without the split, odd with it
+        // (one unit more than its keys': both sides of a cut round down alike, so it
+        // never makes a key); a split needs a positive scale (key_split)
+        run_schedule<false, 1, kLongKeyCost>(
+                     p, NHG, s_pref, s_scan,
+                     [&](int rg) {
+                         const long long v = group_visible<KVM, RM>(p, rg);
+                         const bool split = p.l2scale > 0.0f && group_of<RM>(p, rg).ntok <= kFewTok &&
+                                            v >= (long long)kSplitVarlenKeys * p.F;
+                         return split ? v * kShortKeyCost + 1 : v * kLongKeyCost;
+                     },
+                     [&](int rg, int hg, long long v0, long long v1, bool fin, int slot, long long rk) {
+                         if (uniform((int)rk & 1))
+                             chunk_piece<DT, QM, KVM, P2, RM, 4>(p, smem, pages, uniform(rg), uniform(hg),
                                                                  uniform(v0 / kShortKeyCost),
                                                                  uniform(v1 / kShortKeyCost), uniform((int)fin) != 0,
                                                                  uniform(slot), uniform(rk / kShortKeyCost));
                          else
-                             chunk_piece<DT, QM, KVM, P2, RM, 1>(p, smem, pages, rg, uniform(hg),
+                             chunk_piece<DT, QM, KVM, P2, RM, 1>(p, smem, pages, uniform(rg), uniform(hg),
                                                                  uniform(v0 / kLongKeyCost),
                                                                  uniform(v1 / kLongKeyCost), uniform((int)fin) != 0,
                                                                  uniform(slot), uniform(rk / kLongKeyCost));

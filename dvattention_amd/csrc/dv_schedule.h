@@ -19,7 +19,8 @@ namespace dv {
 // the merge directory (segment -> first partial slot, piece count).  Then
 // piece(row, head_group, v0, v1, final, slot, row_keys) runs for each piece of
 // this workgroup's chunk: visible keys [v0, v1) of the segment (cuts inside a
-// segment fall on multiples of kAlign keys), `final` when
+// segment fall on multiples of kAlign keys; costs, and so v0, v1 and row_keys, may
+// count kUnit parts of a key), `final` when
 // the segment has no other piece, `slot` its partial slot, `row_keys` the row's
 // visible key count.  Slots are
 // sg + workgroup index, increasing along the cost space, so they are unique and
@@ -35,7 +36,7 @@ __device__ inline long long udiv(long long a, long long b) {
 // per-row cost prefix sums: pref_u(r) for a wave-uniform r, pref_v(r) for a
 // per-lane r (called with every lane active), find_row(u) = the last row r
 // with NHG * pref[r] <= u, total = pref[nrows].
-template <int kAlign, class PrefU, class PrefV, class FindRow, class PieceFn>
+template <int kAlign, int kUnit, class PrefU, class PrefV, class FindRow, class PieceFn>
 __device__ inline void split_chunks(const DecodeParams& p, int NHG, long long total, PrefU&& pref_u, PrefV&& pref_v,
                                     FindRow&& find_row, PieceFn&& piece) {
     const int tid = threadIdx.x;
@@ -59,7 +60,11 @@ __device__ inline void split_chunks(const DecodeParams& p, int NHG, long long to
         chunk = (chunk + kAlign - 1) & ~(long long)(kAlign - 1);
         geff = (int)udiv(Wc + chunk - 1, chunk);
     }
-    const long long skew = udiv(chunk * p.skew_pm, 1000);
+    // costs in parts of a key: the cuts fall where they would with keys (cuts between
+    // them put two pieces into some workgroups of short varlen calls: 3 x 1 + 40
+    // tokens, 60 keys 32.2 us, 26.8 so)
+    if (kUnit > 1) chunk = (chunk + kUnit - 1) & ~(long long)(kUnit - 1);
+    const long long skew = udiv(chunk * p.skew_pm, 1000) & ~(long long)(kUnit - 1);
     auto bound = [&](long long i) {
         const long long b = i * chunk + ((i & 1) ? skew : 0);
         return b < Wc ? b : Wc;
@@ -128,7 +133,7 @@ __device__ inline void split_chunks(const DecodeParams& p, int NHG, long long to
     }
 }
 
-template <bool kRegPrefix = false, int kAlign = 1, class RowKeys, class PieceFn>
+template <bool kRegPrefix = false, int kAlign = 1, int kUnit = 1, class RowKeys, class PieceFn>
 __device__ inline void run_schedule(const DecodeParams& p, int NHG, long long* s_pref, long long* s_scan,
                                     RowKeys&& row_keys, PieceFn&& piece) {
     const int tid = threadIdx.x;
@@ -226,7 +231,7 @@ __device__ inline void run_schedule(const DecodeParams& p, int NHG, long long* s
         }
         return lo;
     };
-    split_chunks<kAlign>(p, NHG, total, pref_u, pref_v, find_row, piece);
+    split_chunks<kAlign, kUnit>(p, NHG, total, pref_u, pref_v, find_row, piece);
 }
 
 }  // namespace dv

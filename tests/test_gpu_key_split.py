@@ -53,6 +53,18 @@ def test_varlen_mixed_groups(dv, gpu, dtype, bs, counts, lens):  # noqa: F811
     close(run_varlen(dv, d, 0.1, gpu), O.varlen_paged_sdpa(0.1, **d), dtype, f"{counts}")
 
 
+# keys per view around the number from which a short group's keys are split (96), one
+# view and three, beside a long group
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("lens", [[95], [96], [97], [100, 100, 87], [100, 100, 88], [250, 38, 1]])
+def test_varlen_split_from_96_keys(dv, gpu, dtype, lens):  # noqa: F811
+    counts = [1, 4, 20, 2]
+    W, T, F = len(counts), sum(counts), len(lens)
+    d = rand_varlen(F, W, T, np.concatenate([[0], np.cumsum(counts)]), 2, 16, lens, 64, dtype, seed=sum(lens))
+    d["locations"] = torch.from_numpy(np.repeat(np.array(lens, np.int32)[:, None] - 1, T, axis=1))
+    close(run_varlen(dv, d, 0.1, gpu), O.varlen_paged_sdpa(0.1, **d), dtype, f"{lens}")
+
+
 # views of one, two and more steps of a split (its loads end with the last step), and
 # contiguous views below and above the length from which 5 - 8 tokens are split
 @pytest.mark.parametrize("S", [3, 7])
