@@ -36,7 +36,7 @@ __device__ inline long long udiv(long long a, long long b) {
 // per-row cost prefix sums: pref_u(r) for a wave-uniform r, pref_v(r) for a
 // per-lane r (called with every lane active), find_row(u) = the last row r
 // with NHG * pref[r] <= u, total = pref[nrows].
-template <int kAlign, int kUnit, class PrefU, class PrefV, class FindRow, class PieceFn>
+template <int kAlign, int kUnit, bool kDecode, class PrefU, class PrefV, class FindRow, class PieceFn>
 __device__ inline void split_chunks(const DecodeParams& p, int NHG, long long total, PrefU&& pref_u, PrefV&& pref_v,
                                     FindRow&& find_row, PieceFn&& piece) {
     const int tid = threadIdx.x;
@@ -54,11 +54,41 @@ __device__ inline void split_chunks(const DecodeParams& p, int NHG, long long to
     const long long ng = udiv(Wc + p.min_keys - 1, p.min_keys);
     int geff = Wc == 0 ? 0 : (int)(ng < p.nwg ? ng : p.nwg);
     long long chunk = geff ? udiv(Wc + geff - 1, geff) : 1;
-    if (kAlign > 1 && chunk < 8 * kAlign) {
-        // short chunks: whole stages, or some of them would take one more (one
-        // sequence of 3001 keys in chunks of 68 keys: 18.1 us, of 64: 16.9)
-        chunk = (chunk + kAlign - 1) & ~(long long)(kAlign - 1);
-        geff = (int)udiv(Wc + chunk - 1, chunk);
+    if (kDecode && geff) {
+        const int nseg = nrows * NHG;
+        const long long d0 = pref_u(1);  // the first row's segments' cost
+        // short rows of one length: a workgroup each, as a cut costs a start and the
+        // merge's work.  20 calls, 8 KV heads, pages of 16 keys, cut / whole: 16 rows
+        // of 60 keys 286 / 241 us, of 90 298 / 263, of 200 336 / 338; 64 of 60 / 130
+        // / 200 keys 356 / 265, 493 / 353, 565 / 408; one of 90 / 130 265 / 259, 265 /
+        // 298.  Several views, 4 KV heads, 64 / 1 rows: four of 30 keys 521 / 478, 429
+        // / 469; six of 40 603 / 782, 468 / 715.  Rows of several lengths stay cut:
+        // no cut of equal costs falls between them (16 of 7-60 keys 281 / 351 us).
+        const int lim = nseg < 64 ? 96 : p.F == 1 ? 256 : 128;
+        if (chunk < d0 && d0 <= c + lim && d0 * nrows == total) {
+            bool same = true;
+            if (nrows <= kWave) {  // every wave by itself
+                const int r = tid & (kWave - 1);
+                const long long before = pref_v(r < nrows ? r : 0);
+                same = ballot(r < nrows && before != r * d0) == 0;
+            } else {
+                for (int r0 = 0; r0 < nrows; r0 += nthreads) {
+                    const int r = r0 + tid;
+                    same = same && (r >= nrows || pref_v(r) == r * d0);
+                }
+                same = __syncthreads_and(same) != 0;
+            }
+            if (same) {
+                chunk = d0;
+                geff = nseg;
+            }
+        }
+        // short chunks of longer rows: whole stages, or some of them would take one
+        // more (one sequence of 3001 keys in chunks of 68 keys: 18.1 us, of 64: 16.9)
+        if (kAlign > 1 && chunk * nseg < Wc && chunk < 8 * kAlign) {
+            chunk = (chunk + kAlign - 1) & ~(long long)(kAlign - 1);
+            geff = (int)udiv(Wc + chunk - 1, chunk);
+        }
     }
     // costs in parts of a key: the cuts fall where they would with keys (cuts between
     // them put two pieces into some workgroups of short varlen calls: 3 x 1 + 40
@@ -133,7 +163,7 @@ __device__ inline void split_chunks(const DecodeParams& p, int NHG, long long to
     }
 }
 
-template <bool kRegPrefix = false, int kAlign = 1, int kUnit = 1, class RowKeys, class PieceFn>
+template <bool kRegPrefix = false, int kAlign = 1, int kUnit = 1, bool kDecode = false, class RowKeys, class PieceFn>
 __device__ inline void run_schedule(const DecodeParams& p, int NHG, long long* s_pref, long long* s_scan,
                                     RowKeys&& row_keys, PieceFn&& piece) {
     const int tid = threadIdx.x;
@@ -231,7 +261,7 @@ __device__ inline void run_schedule(const DecodeParams& p, int NHG, long long* s
         }
         return lo;
     };
-    split_chunks<kAlign, kUnit>(p, NHG, total, pref_u, pref_v, find_row, piece);
+    split_chunks<kAlign, kUnit, kDecode>(p, NHG, total, pref_u, pref_v, find_row, piece);
 }
 
 }  // namespace dv

@@ -57,3 +57,17 @@ def test_paged_many_views(dv, gpu, dtype, F, bs):  # noqa: F811
     loc[64:] = -1  # no view of the later blocks is seen
     d = rand_paged(F, 3, 1, 4, bs, list(lens), 32, dtype, seed=bs, loc=loc)
     close(run_paged(dv, d, 0.1, gpu), O.paged_sdpa(0.1, **d), dtype, f"F={F}, first block only")
+
+
+# short rows, which get a workgroup each where all have one length: lengths up to and
+# past the limits of that (96, 128 and 256 keys), more and fewer than 64 rows, one row
+# of another length among them
+@pytest.mark.parametrize("W,Hkv", [(3, 2), (20, 8), (70, 4)])
+@pytest.mark.parametrize("lens", [[1], [60], [96], [97], [130], [256], [257], [40, 60], [100, 29]])
+@pytest.mark.parametrize("odd", [None, 0, 1])
+def test_paged_short_rows(dv, gpu, W, Hkv, lens, odd):  # noqa: F811
+    loc = np.array(lens)[:, None, None] - 1 + np.zeros((len(lens), W, 1), int)
+    if odd is not None:
+        loc[-1, odd] -= 1
+    d = rand_paged(len(lens), W, 1, Hkv, 16, lens, 64, torch.bfloat16, seed=W, loc=loc)
+    close(run_paged(dv, d, 0.1, gpu), O.paged_sdpa(0.1, **d), torch.bfloat16, f"W={W} {lens} {odd}")
